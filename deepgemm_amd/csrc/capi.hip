@@ -699,6 +699,22 @@ int mmoe_marlin_pack(void* out, const void* in, int64_t groups, int64_t rows, in
              : MMOE_ERR_HIP;
 }
 
+int mmoe_cast_fp8_marlin(void* out_fp8, float* out_scale, const void* w_bf16, int64_t groups,
+                         int64_t rows, int64_t k, void* stream) {
+  if (groups < 0 || rows < 0 || k <= 0) return MMOE_ERR_ARGUMENT;
+  if (rows % 16 || k % 16) return MMOE_ERR_MARLIN_DIVISIBLE;
+  if (k > mmoe::kCastMaxCols) return MMOE_ERR_UNSUPPORTED_SHAPE;
+  if (groups * rows == 0) return MMOE_OK;
+  if (out_fp8 == nullptr || out_scale == nullptr || w_bf16 == nullptr) return MMOE_ERR_NULL_POINTER;
+  if (reinterpret_cast<uintptr_t>(out_fp8) % 16 || reinterpret_cast<uintptr_t>(w_bf16) % 16)
+    return MMOE_ERR_ARGUMENT;
+  return mmoe::launch_cast_marlin(static_cast<uint8_t*>(out_fp8), out_scale,
+                                  static_cast<const uint16_t*>(w_bf16), groups, rows, k,
+                                  static_cast<hipStream_t>(stream)) == hipSuccess
+             ? MMOE_OK
+             : MMOE_ERR_HIP;
+}
+
 int mmoe_debug_f32_to_e4m3(uint8_t* out, const float* in, int64_t n, void* stream) {
   if (n < 0) return MMOE_ERR_ARGUMENT;
   if (n == 0) return MMOE_OK;

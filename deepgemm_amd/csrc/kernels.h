@@ -245,6 +245,11 @@ hipError_t launch_gather_tasks(uint8_t* grouped_x, float* grouped_scale, const u
 
 hipError_t launch_cast_fp8_channelwise(uint8_t* out, float* scale, const uint16_t* x,
                                        int64_t rows, int64_t cols, hipStream_t stream);
+// The cast and the Marlin pack of grouped weights [groups, rows, k] in one pass (rows % 16 == 0,
+// k % 16 == 0, k <= kCastMaxCols, x and out 16-byte aligned).
+constexpr int kCastMaxCols = 8192;  // a row's values stay in registers up to here
+hipError_t launch_cast_marlin(uint8_t* out, float* scale, const uint16_t* x, int64_t groups,
+                              int64_t rows, int64_t k, hipStream_t stream);
 hipError_t launch_marlin_pack(uint8_t* out, const uint8_t* in, int64_t groups, int64_t rows,
                               int64_t k, hipStream_t stream);
 hipError_t launch_f32_to_e4m3(uint8_t* out, const float* in, int64_t n, hipStream_t stream);

@@ -151,8 +151,34 @@ def weight8bit_nt_kpack2_marlin(weight: torch.Tensor, k_tile: int = 16,
             .permute(0, 1, 3, 2, 4).contiguous().reshape(num_groups, rows // n_tile, k * n_tile))
 
 
+_CAST_MARLIN_MAX_K = 8192  # the one-pass kernel holds a row's values in registers up to here
+
+
+def _one_pass_transform(w: torch.Tensor) -> bool:
+    """Whether ``mmoe_cast_fp8_marlin`` takes this weight (any other goes through the cast and the
+    pack one after the other, which also raise what is wrong with it)."""
+    return (w.dim() == 3 and w.is_cuda and w.dtype == torch.bfloat16 and w.numel() > 0
+            and w.size(1) % 16 == 0 and w.size(2) % 16 == 0 and w.size(2) <= _CAST_MARLIN_MAX_K)
+
+
+def _cast_marlin(weights: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+    w = weights.contiguous()
+    if w.data_ptr() % 16:
+        w = w.clone()
+    g, rows, k = w.shape
+    packed = torch.empty((g, rows // 16, k * 16), dtype=torch.float8_e4m3fn, device=w.device)
+    scale = torch.empty((g, rows), dtype=torch.float32, device=w.device)
+    _capi.check(_capi.load().mmoe_cast_fp8_marlin(packed.data_ptr(), scale.data_ptr(), w.data_ptr(),
+                                                  g, rows, k, _stream_handle()),
+                "transform_fp8_weights_for_mega_moe")
+    return packed, scale
+
+
 def transform_fp8_weights_for_mega_moe(l1_weights: torch.Tensor, l2_weights: torch.Tensor):
-    """megamoe/__init__.py:280-289."""
+    """megamoe/__init__.py:280-289. bf16 weights on the GPU go through one kernel that casts and
+    packs in one pass (bitwise the cast followed by the pack)."""
+    if _one_pass_transform(l1_weights) and _one_pass_transform(l2_weights):
+        return _cast_marlin(l1_weights), _cast_marlin(l2_weights)
     l1_fp8, l1_scale = cast_grouped_weight_to_fp8_channelwise(l1_weights)
     l2_fp8, l2_scale = cast_grouped_weight_to_fp8_channelwise(l2_weights)
     return ((weight8bit_nt_kpack2_marlin(l1_fp8), l1_scale),

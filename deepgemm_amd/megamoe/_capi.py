@@ -118,6 +118,7 @@ SIGNATURES = {
         ctypes.c_int, [c_p] * 5 + [ctypes.c_int] * 5 + [c_p]),
     "mmoe_cast_fp8_channelwise": (ctypes.c_int, [c_p, c_p, c_p, c_i64, c_i64, c_p]),
     "mmoe_marlin_pack": (ctypes.c_int, [c_p, c_p, c_i64, c_i64, c_i64, c_p]),
+    "mmoe_cast_fp8_marlin": (ctypes.c_int, [c_p, c_p, c_p, c_i64, c_i64, c_i64, c_p]),
     "mmoe_debug_f32_to_e4m3": (ctypes.c_int, [c_p, c_p, c_i64, c_p]),
 }
 

@@ -289,6 +289,12 @@ int mmoe_cast_fp8_channelwise(void* out_fp8, float* out_scale, const void* x_bf1
 int mmoe_marlin_pack(void* out, const void* in, int64_t groups, int64_t rows, int64_t k,
                      void* stream);
 
+/* Both at once for grouped bf16 weights [G, R, K] (R and K multiples of 16, K <= 8192, both
+ * pointers 16-byte aligned): out_fp8 e4m3 [G, R/16, K*16], out_scale f32 [G, R]; the bytes of
+ * mmoe_cast_fp8_channelwise followed by mmoe_marlin_pack, in one pass over the weights. */
+int mmoe_cast_fp8_marlin(void* out_fp8, float* out_scale, const void* w_bf16, int64_t groups,
+                         int64_t rows, int64_t k, void* stream);
+
 /* Elementwise f32 -> e4m3fn (saturating RNE after a clip to +-448, the conversion every
  * quantising kernel here uses); exposed so the conversion can be checked exhaustively. */
 int mmoe_debug_f32_to_e4m3(uint8_t* out, const float* in, int64_t n, void* stream);

@@ -57,6 +57,67 @@ def test_marlin_pack_bitwise(mm, cuda):
     assert torch.equal(got.view(torch.uint8), O.marlin_pack(w).view(torch.uint8))
 
 
+@pytest.mark.parametrize("cols", [8, 512, 2048, 2056, 4096, 4104, 7168, 8192, 8200, 1022])
+def test_cast_fp8_channelwise_every_kernel(mm, cuda, cols):
+    """Row widths on both sides of each kernel's limit (2048, 4096, 8192 columns; not a multiple of
+    8), aligned and as an unaligned view (the kernel that reads values one by one): every finite
+    bf16 value against the oracle's division, bitwise, and rows with infinities, NaN and signed
+    zeros the same from both kernels."""
+    bits = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    finite = bits[torch.isfinite(bits)]
+    finite = finite[finite.abs() < 2.0 ** 120]
+    rows = min(200, -(-finite.numel() // cols))
+    gen = torch.Generator().manual_seed(cols)
+    # ascending in magnitude, so that a row's values span few binades and fill the codes
+    finite = finite[finite.abs().float().argsort()]
+    x = finite[torch.arange(rows * cols) * finite.numel() // (rows * cols)].view(rows, cols).clone()
+    x = torch.cat([x, (torch.randn((3, cols), generator=gen)).to(torch.bfloat16)])
+    log(f"cast cols={cols}: {x.shape[0]} rows")
+    qr, sr = O.cast_to_fp8_channelwise(x)
+    pad = torch.empty((x.numel() + 1,), dtype=torch.bfloat16, device=cuda)
+    view = pad[1:].view(x.shape)
+    view.copy_(x)
+    for name, t in (("aligned", x.to(cuda)), ("unaligned", view)):
+        q, s = mm.cast_to_fp8_channelwise(t)
+        assert torch.equal(s.cpu(), sr), name
+        assert torch.equal(q.cpu().view(torch.uint8), qr.view(torch.uint8)), name
+    special = (torch.randn((4, cols), generator=gen)).to(torch.bfloat16)
+    special[0, 0] = float("inf")
+    special[1, cols - 1] = float("-inf")
+    special[2, cols // 2] = float("nan")
+    special[3, ::2] = -0.0
+    pad = torch.empty((special.numel() + 1,), dtype=torch.bfloat16, device=cuda)
+    view = pad[1:].view(special.shape)
+    view.copy_(special)
+    q, s = mm.cast_to_fp8_channelwise(special.to(cuda))
+    qv, sv = mm.cast_to_fp8_channelwise(view)
+    assert torch.equal(q.view(torch.uint8), qv.view(torch.uint8)) and torch.equal(s, sv)
+    assert torch.isinf(s[:2]).all() and torch.isfinite(s[2:]).all()
+    assert torch.all((q[0, 1:].view(torch.uint8) & 0x7f) == 0), "finite values beside an infinity"
+    assert torch.all(q[3, ::2].view(torch.uint8) == 0x80), "negative zeros"
+
+
+@pytest.mark.parametrize("shape", [(1, 16, 16), (2, 48, 144), (3, 32, 2048), (1, 16, 2064), (2, 16, 4096),
+                                   (1, 32, 4112), (1, 16, 7168), (1, 16, 8192), (1, 16, 8208)])
+def test_transform_weights_bitwise(mm, cuda, shape):
+    """Casting straight into the Marlin layout (up to 8192 columns; above, the cast and the pack one
+    after the other) against the oracle's cast and pack, from contiguous weights, a strided and an
+    unaligned view."""
+    gen = torch.Generator().manual_seed(sum(shape))
+    w = (torch.randn(shape, generator=gen) * 0.1).to(torch.bfloat16)
+    w[0, 3] = 0.0
+    (ref, ref_s), _ = O.transform_fp8_weights_for_mega_moe(w, w)
+    strided = torch.empty(shape[:2] + (shape[2] + 8,), dtype=torch.bfloat16, device=cuda)[..., :shape[2]]
+    strided.copy_(w)
+    odd = torch.empty((w.numel() + 1,), dtype=torch.bfloat16, device=cuda)[1:].view(shape)
+    odd.copy_(w)
+    log(f"transform {shape}")
+    for a, b in ((w.to(cuda), strided), (odd, w.to(cuda))):
+        for got, got_s in mm.transform_fp8_weights_for_mega_moe(a, b):
+            assert got.shape == ref.shape and torch.equal(got_s.cpu(), ref_s)
+            assert torch.equal(got.cpu().view(torch.uint8), ref.view(torch.uint8))
+
+
 # ------------------------------------------------------------------ routing
 ROUTE_CASES = {
     # name: (S, E, K, global experts or "zipf"/"invalid")
