@@ -455,7 +455,7 @@ int mmoe_forward_stages(const mmoe_forward_args* a, int first_stage, int last_st
     p.direct_flag = direct_flag;
     p.pipe = at<int32_t>(ws, l.pipe_offset);
     p.spin_limit = (a->debug_flags & MMOE_DEBUG_NO_WAIT) != 0 ? 0 : mmoe::kPipeSpinLimit;
-    if (runs(MMOE_STAGE_COMBINE) && a->hidden % 8 == 0 && a->hidden <= mmoe::kPipeCombineMaxHidden) {
+    if (runs(MMOE_STAGE_COMBINE) && a->hidden % 8 == 0) {
       p.y = static_cast<uint16_t*>(a->y);
       combined = true;
     }

@@ -59,12 +59,13 @@ constexpr int kGemmWaves = kGemmThreads / kWave;
 constexpr int kMaxGemmExperts = 256;
 // STREAM engine
 constexpr int kStreamUnit = 64;     // output columns per wave
-constexpr int kStreamRows = 64;     // rows of a decode pipeline group
+constexpr int kStreamRows = 64;     // rows of a decode pipeline GEMM2 item
 constexpr int kStreamItemRows = 128;  // rows of a STREAM item of the 8-wave GEMM kernel
 constexpr int kStreamAutoMaxRows = kStreamItemRows;  // the auto schedule streams experts up to this
 constexpr int kStreamDepth = 4;     // 64-k weight steps in flight per wave
 constexpr int kAChunk = 65536;      // bytes of one A chunk buffer (32*MT rows x 2048/MT k)
 constexpr int kALoads = kAChunk / 1024 / kGemmWaves;  // 16-byte A loads per lane per chunk
+constexpr int kNarrowDepth = 8;     // weight steps in flight of a narrow item's waves
 // TILE engine: 256 x 256 output tile, BK = 128, the 8 waves as 2 (M) x 4 (N), each wave 128
 // rows x 64 columns (4 x 2 MFMA tiles of 32 x 32)
 constexpr int kTileBM = 256, kTileBN = 256, kTileBK = 128;
@@ -208,13 +209,33 @@ __device__ __forceinline__ void publish_tile_scales(TileTables& tt, const TileSc
 // SwiGLU: y is stored in bf16 (the reference fused path's rounding of the activation before
 // its quantization). kPmax (the decode pipeline's GEMM1): the row maxima of the rounded values
 // are stored as well.
+// The stores go through a buffer descriptor of the tile's mrows rows, whose bounds check drops the
+// rows past them: no branch a row (at 4 row tiles 64 of them, which had also kept the compiler
+// from inlining the tile in a kernel of many variants).
+constexpr int kBufferFlags = 0x00020000;  // raw buffer, 32-bit data format (unused by raw accesses)
+template <typename T>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(T* p, int64_t first, int64_t count) {
+  // (uniform in the wave: the descriptor sits in scalar registers)
+  const int64_t at = reinterpret_cast<int64_t>(p + first);
+  const int lo = __builtin_amdgcn_readfirstlane(static_cast<int>(at));
+  const int hi = __builtin_amdgcn_readfirstlane(static_cast<int>(at >> 32));
+  const int bytes = __builtin_amdgcn_readfirstlane(static_cast<int>(count < 0 ? 0 : count) * static_cast<int>(sizeof(T)));
+  void* base = reinterpret_cast<void*>(static_cast<int64_t>(hi) << 32 | static_cast<uint32_t>(lo));
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, kBufferFlags);
+}
+
 template <bool kSwiglu, int MT, bool kPmax = false, bool kCoherent = false>
 __device__ __forceinline__ void store_tile(const GemmArgs& g, const v16f (&acc)[MT][2], int row0,
                                            int mrows, int unit, const TileTables& tt, int trow0) {
+  constexpr int kAux = kCoherent ? 16 : 0;  // sc1
   const int tid = opaque_tid();
   const int lane = tid & (kWave - 1), wave = tid / kWave;
   const int rl = lane & 31, hk = lane >> 5;
   const float b0 = tt.bs[wave][0][lane], b1 = tt.bs[wave][1][lane];
+  const int cols = kSwiglu ? g.sw.inter : g.n;  // of an output row
+  const __amdgpu_buffer_rsrc_t out =
+      tile_rows(kSwiglu ? g.sw.y : g.c, static_cast<int64_t>(row0) * cols, static_cast<int64_t>(mrows) * cols);
+  const int at = (hk * 4 * cols + unit * (kSwiglu ? 32 : 64) + rl) * 2;  // the lane's row 0 and first column
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     // the 16 rows' table entries read at once (rows past mrows read entries never used)
@@ -228,28 +249,14 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const v16f (&acc)[
     float pm[16];  // kPmax: |y| of the lane's channel in each of its 16 rows
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      pm[v] = 0.0f;
-      const int r = mt * 32 + (v >> 2) * 8 + hk * 4 + (v & 3);
-      if (r >= mrows) continue;
+      const int off = at + (mt * 32 + (v >> 2) * 8 + (v & 3)) * cols * 2;
       if (!kSwiglu) {
-        uint16_t* crow = g.c + static_cast<int64_t>(row0 + r) * g.n + unit * 64 + rl;
-        const uint16_t c0 = f32_to_bf16(acc[mt][0][v] * xs[v] * b0);
-        const uint16_t c1 = f32_to_bf16(acc[mt][1][v] * xs[v] * b1);
-        if constexpr (kCoherent) {
-          __hip_atomic_store(crow, c0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          __hip_atomic_store(crow + 32, c1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-          crow[0] = c0;
-          crow[32] = c1;
-        }
+        __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(acc[mt][0][v] * xs[v] * b0), out, off, 0, kAux);
+        __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16(acc[mt][1][v] * xs[v] * b1), out, off + 64, 0, kAux);
       } else {
         const float yv = swiglu_value(g, acc[mt][0][v], acc[mt][1][v], xs[v], b0, b1, rw[v]);
-        const int64_t at = static_cast<int64_t>(row0 + r) * g.sw.inter + unit * 32 + rl;
         const uint16_t yb = f32_to_bf16(yv);
-        if constexpr (kCoherent)
-          __hip_atomic_store(g.sw.y + at, yb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        else
-          g.sw.y[at] = yb;
+        __builtin_amdgcn_raw_buffer_store_b16(yb, out, off, 0, kAux);
         if constexpr (kPmax) pm[v] = fabsf(bf16_to_f32(yb));
       }
     }
@@ -263,7 +270,9 @@ __device__ __forceinline__ void store_tile(const GemmArgs& g, const v16f (&acc)[
       for (int v = 1; v < 16; ++v) mv = (rl & 15) == v ? pm[v] : mv;
       const int v = rl & 15;
       const int r = mt * 32 + (v >> 2) * 8 + hk * 4 + (v & 3);
-      if (rl >= 16 && r < mrows) g.row_pmax[static_cast<int64_t>(row0 + r) * (g.n / kStreamUnit) + unit] = mv;
+      if (rl >= 16 && r < mrows)
+        __hip_atomic_store(g.row_pmax + static_cast<int64_t>(row0 + r) * (g.n / kStreamUnit) + unit, mv,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
 }
@@ -287,13 +296,30 @@ __device__ __forceinline__ void lds_barrier() {
 // same k of 8 consecutive rows hit 8 distinct 16-byte bank groups.
 __device__ __forceinline__ int swizzle_piece(int p, int r) { return (p & ~7) | ((p ^ r) & 7); }
 
-// One workgroup tile (expert e, 512-column block nb, rows [row0, row0 + mrows), mrows <= 32*MT)
-// over the full K. kFast: K is a multiple of the chunk (2048/MT k), ring 4 steps deep (2 for
-// four row tiles, whose 128 accumulators leave no room for more); else 128-k chunks and a
-// one-step ring (small shapes).
+// An A chunk in LDS: 32*MT rows of kc k-bytes, kc <= kMaxK, at a row stride of kMaxK. Piece i of a
+// lane is 16 bytes of row row(i, ..) at piece position pos(i, ..): 64 lanes cover a row's 1024
+// bytes (MT = 4: two rows' 512), whole 128-byte lines. A position past kc is never read; the piece
+// put there is the chunk's last one (src), so that loads and LDS writes need no masks.
+template <int MT, int kLoads = kALoads>
+struct AChunk {
+  static constexpr int kBytes = kLoads * kGemmWaves * 1024;
+  static constexpr int kMaxK = kBytes / (32 * MT);
+  static constexpr int kPieces = kMaxK / 16;  // piece positions of a row
+  static __device__ __forceinline__ int row(int i, int lane, int wave) {
+    return (i * kWave + lane) / kPieces * kGemmWaves + wave;
+  }
+  static __device__ __forceinline__ int pos(int i, int lane) { return (i * kWave + lane) % kPieces; }
+  // the piece of the chunk at that position (swizzled by the row)
+  static __device__ __forceinline__ int src(int i, int lane, int wave, int kc) {
+    return swizzle_piece(min(pos(i, lane), kc / 16 - 1), row(i, lane, wave));
+  }
+};
+
+// One workgroup tile (expert e, column block nb of `waves` 64-column units, rows [row0, row0 +
+// mrows), mrows <= 32*MT) over the full K in chunks of kc k-bytes (GemmArgs::kc: at most 2048/MT, a
+// multiple of 64*D that divides K), with a ring of D weight steps a wave.
 //
-// A chunk c+1 is loaded into registers (8 x 16 bytes per lane, whole 128-byte lines: lane l of
-// load i covers LDS bytes gi*1024 + 16*l of the chunk buffer, gi = 8i + wave) right after the
+// A chunk c+1 is loaded into registers (kLoads x 16 bytes per lane, AChunk's pieces) right after the
 // barrier that opens chunk c, and written to its LDS buffer at the end of chunk c, before the
 // next barrier. Plain loads keep the memory counter in order, so every wait the compiler places
 // for a weight step or for the staged chunk is exact; the chunk's loads are older than all
@@ -303,58 +329,73 @@ __device__ __forceinline__ int swizzle_piece(int p, int r) { return (p & ~7) | (
 // pipeline's wait for the item's rows), then the item's scales and A rows are loaded.
 // kAResident: before_a also leaves the item's whole A in the LDS chunk buffers (K of at most two
 // chunks), so no A rows are loaded here.
+// kNarrow: only the first `waves` waves have columns (2 or 4 of the 8); the others help with A
+// and leave. A ring of 8 steps then keeps enough bytes in flight, and the few waves need no
+// barrier a step.
 struct NoHook {
   __device__ __forceinline__ void operator()() const {}
 };
-template <bool kGather, bool kSwiglu, int MT, bool kFast, bool kEarly = false, bool kAResident = false,
-          bool kPmax = false, bool kCoherent = false, typename Hook = NoHook>
+template <bool kGather, bool kSwiglu, int MT, int D, bool kEarly = false, bool kAResident = false,
+          bool kPmax = false, bool kCoherent = false, bool kNarrow = false, int kLoads = kALoads,
+          typename Hook = NoHook>
 __device__ void stream_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, int mrows, int nb,
-                            uint8_t* smem, TileTables& tt, const Hook& before_a = Hook{}) {
-  static_assert(!kAResident || (kEarly && kFast), "a resident A is staged by the hook");
-  // four row tiles: the accumulators take the registers of two ring steps
-  constexpr int D = kFast ? (MT == 4 ? kStreamDepth / 2 : kStreamDepth) : 1;
-  constexpr int kFullChunk = kAChunk / (32 * MT);  // k-bytes per chunk
-  const int kc = kFast ? kFullChunk : 128;
+                            int kc, uint8_t* smem, TileTables& tt, const Hook& before_a = Hook{},
+                            int waves = kGemmWaves) {
+  static_assert(!kAResident || kEarly, "a resident A is staged by the hook");
+  using Chunk = AChunk<MT, kLoads>;
   const int spc = kc / 64;  // steps per chunk
   const int nchunks = g.k / kc;
   const int tid = opaque_tid();
   const int lane = tid & (kWave - 1);
   const int wave = tid / kWave;
   const int units = g.n / kStreamUnit;
-  const int unit_raw = nb * kGemmWaves + wave;
+  const int unit_raw = nb * (kNarrow ? waves : kGemmWaves) + wave;
   const bool active = unit_raw < units;  // a partial column block leaves waves without columns
   const int unit = active ? unit_raw : units - 1;
 
-  const int chunk_bytes = 32 * MT * kc;
-  const uint8_t* asrc[kALoads];
+  const uint8_t* asrc[kLoads];
   auto a_sources = [&]() {  // (reads the row table: after before_a, which may fill it)
 #pragma unroll
-    for (int i = 0; i < kALoads; ++i) {
-      const int pos = (i * kGemmWaves + wave) * 1024 + lane * 16;
-      const int r = pos / kc;
-      const int p = swizzle_piece((pos - r * kc) >> 4, r);
-      asrc[i] = a_row_ptr<kGather>(g, rs, row0 + (r < mrows ? r : 0)) + p * 16;
+    for (int i = 0; i < kLoads; ++i) {
+      const int r = Chunk::row(i, lane, wave);
+      asrc[i] = a_row_ptr<kGather>(g, rs, row0 + (r < mrows ? r : 0)) + Chunk::src(i, lane, wave, kc) * 16;
     }
   };
   if constexpr (!kEarly) a_sources();
-  int4 astage[kALoads];
+  int4 astage[kLoads];
   auto load_chunk = [&](int chunk) {
     if constexpr (kAResident) return;
 #pragma unroll
-    for (int i = 0; i < kALoads; ++i)
-      if (kFast || (i * kGemmWaves + wave) * 1024 < chunk_bytes)
-        astage[i] = ld16(asrc[i] + static_cast<int64_t>(chunk) * kc);
+    for (int i = 0; i < kLoads; ++i) astage[i] = ld16(asrc[i] + static_cast<int64_t>(chunk) * kc);
   };
   auto store_chunk = [&](int chunk) {
     if constexpr (kAResident) return;
-    uint8_t* dst = smem + (chunk & 1) * kAChunk + wave * 1024 + lane * 16;
+    uint8_t* dst = smem + (chunk & 1) * Chunk::kBytes;
 #pragma unroll
-    for (int i = 0; i < kALoads; ++i)
-      if (kFast || (i * kGemmWaves + wave) * 1024 < chunk_bytes)
-        *reinterpret_cast<int4*>(dst + i * kGemmWaves * 1024) = astage[i];
+    for (int i = 0; i < kLoads; ++i)
+      *reinterpret_cast<int4*>(dst + Chunk::row(i, lane, wave) * Chunk::kMaxK + Chunk::pos(i, lane) * 16) = astage[i];
   };
+  if constexpr (kNarrow) {
+    if (__builtin_amdgcn_readfirstlane(wave) >= waves) {  // no columns: this wave's share of A, in step with the others' barriers
+      if constexpr (kEarly) {
+        before_a();
+        if constexpr (!kAResident) a_sources();
+      }
+      const TileScaleRegs tsr = load_tile_scales<kGather, kSwiglu>(g, rs, e, row0, kAResident ? 0 : mrows, 0);
+      load_chunk(0);
+      store_chunk(0);
+      publish_tile_scales(tt, tsr, kAResident ? 0 : mrows);
+      lds_barrier();
+      for (int c = 0; c + 1 < nchunks; ++c) {
+        load_chunk(c + 1);
+        store_chunk(c + 1);
+        lds_barrier();
+      }
+      return;
+    }
+  }
   // operand reads: lane l is row l%32 (+32 mt), k-bytes [64j + 32*(l/32), +32) of chunk step j
-  const uint8_t* sbase = smem + (lane & 31) * kc;
+  const uint8_t* sbase = smem + (lane & 31) * Chunk::kMaxK;
   const int hk = lane >> 5;
   int pc[2][2];  // swizzled byte offset of piece 4v + 2hk + h within its 128-byte group
 #pragma unroll
@@ -389,16 +430,17 @@ __device__ void stream_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0
   auto compute = [&](int d, int c, int j) {
     const v8i b0 = make_v8i(br[d][0][0], br[d][0][1]);
     const v8i b1 = make_v8i(br[d][1][0], br[d][1][1]);
-    const uint8_t* base = sbase + (c & 1) * kAChunk + (j >> 1) * 128;
+    const uint8_t* base = sbase + (c & 1) * Chunk::kBytes + (j >> 1) * 128;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      const uint8_t* rb = base + mt * 32 * kc;
-      const v8i a = make_v8i(*reinterpret_cast<const int4*>(rb + pc[j & 1][0]),
-                             *reinterpret_cast<const int4*>(rb + pc[j & 1][1]));
+      const uint8_t* rb = base + mt * 32 * Chunk::kMaxK;
+      const v8i a = make_v8i(*reinterpret_cast<const int4*>(rb + pc[d & 1][0]),
+                             *reinterpret_cast<const int4*>(rb + pc[d & 1][1]));
       acc[mt][0] = mfma_fp8(a, b0, acc[mt][0]);
       acc[mt][1] = mfma_fp8(a, b1, acc[mt][1]);
     }
   };
+  static_assert(D % 2 == 0, "ring slot d holds steps of d's parity");
 
   if constexpr (kEarly) {
 #pragma unroll
@@ -432,7 +474,7 @@ __device__ void stream_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0
         compute(d, c, j + d);
         issue(d, c * spc + j + d + D);
         __builtin_amdgcn_sched_barrier(0);
-        if (kFast) step_barrier();
+        if (!kNarrow) step_barrier();
       }
     }
     store_chunk(c + 1);  // its buffer was last read in chunk c - 1, before the last barrier
@@ -446,7 +488,7 @@ __device__ void stream_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0
         compute(d, c, j + d);
         issue(d, c * spc + j + d + D);
         __builtin_amdgcn_sched_barrier(0);
-        if (kFast) step_barrier();
+        if (!kNarrow) step_barrier();
       }
     }
 #pragma unroll
@@ -1223,9 +1265,9 @@ __device__ __forceinline__ void tile_coords(int local, int cnt, int tile_nb, int
   mt = group * 4 + (in_group - nb * rows_in_group);
 }
 
-// kAnyK: K not a multiple of the STREAM chunk (small shapes); the production shapes compile
-// without those variants, which keeps the kernel's code (and its cold instruction fetches in
-// the one-time prologue) smaller.
+// kAnyK: K whose STREAM chunks do not take the 4-step weight ring (K not a multiple of 256); the
+// other shapes compile without those variants, which keeps the kernel's code (and its cold
+// instruction fetches in the one-time prologue) smaller.
 // A dual launch's kernel that the routed rows do not select returns at once (GemmArgs).
 __device__ __forceinline__ bool dual_skips(const GemmArgs& g, bool wide) {
   return g.dual_rows != nullptr && ((*g.dual_rows >= g.dual_min_rows) != wide);
@@ -1291,9 +1333,6 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs 
   }
   const int total = s_prefix[E];
   const int tile_nb = (g.n + kTileBN - 1) / kTileBN;
-  const bool fast1 = !kAnyK || g.k % (kAChunk / 32) == 0;
-  const bool fast2 = !kAnyK || g.k % (kAChunk / 64) == 0;
-  const bool fast4 = !kAnyK || g.k % (kAChunk / 128) == 0;
   const ItemDeal deal = deal_items(total);
   // the route weights cached in LDS are valid until the first item's loads overwrite them
   const float* task_w = reinterpret_cast<const float*>(smem);
@@ -1336,14 +1375,13 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs 
         rs = RowSrc{s_tok, s_rw, row0};
       }
       if (mrows > 64) {
-        if (fast4) stream_tile<kGather, kSwiglu, 4, true>(g, rs, e, row0, mrows, nb, smem, s_tt);
-        else if (kAnyK) stream_tile<kGather, kSwiglu, 4, false>(g, rs, e, row0, mrows, nb, smem, s_tt);
+        stream_tile<kGather, kSwiglu, 4, 2>(g, rs, e, row0, mrows, nb, g.kc[2], smem, s_tt);
       } else if (mrows > 32) {
-        if (fast2) stream_tile<kGather, kSwiglu, 2, true>(g, rs, e, row0, mrows, nb, smem, s_tt);
-        else if (kAnyK) stream_tile<kGather, kSwiglu, 2, false>(g, rs, e, row0, mrows, nb, smem, s_tt);
+        if (!kAnyK || g.ring[1] == 4) stream_tile<kGather, kSwiglu, 2, 4>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
+        else if (kAnyK) stream_tile<kGather, kSwiglu, 2, 2>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
       } else {
-        if (fast1) stream_tile<kGather, kSwiglu, 1, true>(g, rs, e, row0, mrows, nb, smem, s_tt);
-        else if (kAnyK) stream_tile<kGather, kSwiglu, 1, false>(g, rs, e, row0, mrows, nb, smem, s_tt);
+        if (!kAnyK || g.ring[0] == 4) stream_tile<kGather, kSwiglu, 1, 4>(g, rs, e, row0, mrows, nb, g.kc[0], smem, s_tt);
+        else if (kAnyK) stream_tile<kGather, kSwiglu, 1, 2>(g, rs, e, row0, mrows, nb, g.kc[0], smem, s_tt);
       }
     }
     __syncthreads();
@@ -1356,23 +1394,26 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs 
 // instead of after the slowest XCD's last GEMM1 item, and without the requant's and GEMM2's
 // launches and prologues.
 //
-// Work: the routed rows are cut into groups (an expert's rows in chunks of kStreamRows); a group
-// has n1 GEMM1 items and n2 GEMM2 items (512-column blocks). The groups are dealt to the XCDs in
-// contiguous ranges, and the workgroups of an XCD -- found by the hardware XCD id, not by launch
-// order -- claim its queue in order: every GEMM1 item of its groups, then their GEMM2 items. A
-// claim goes out one item ahead, so its latency hides behind an item.
+// Work: an expert's rows are cut into groups, a GEMM1 item is a group and a column block (512
+// columns, fewer when there are few groups: PipeShape), and a GEMM2 item a column block and the rows
+// of a group or of half of one. All the GEMM1 items in expert order are dealt to the XCDs in equal
+// contiguous ranges, and so are the GEMM2 items; the workgroups of an XCD -- found by the hardware XCD id, not
+// by launch order -- claim their range of GEMM1 items, then of GEMM2 items, in order. A claim goes
+// out one item ahead, so its latency hides behind an item. A workgroup whose range is all claimed
+// takes items of the other XCDs' ranges.
 //
-// Hand-off, inside the XCD, whose CUs share its L2 (the per-CU L1 is write-through): a GEMM1
-// item waits for its bf16 SwiGLU stores (vmcnt 0) and counts itself done for its group. A GEMM2
-// item issues its first weight steps, polls until its group's count is complete, invalidates
-// its CU's L1 and requantizes the group's rows from L2 straight into its LDS A buffers (the
+// Hand-off: a GEMM1 item stores its bf16 SwiGLU rows and their block maxima device-coherent (sc1,
+// through its XCD's L2), waits for them (vmcnt 0) and counts itself done for its group. A GEMM2
+// item, of any XCD, issues its first weight steps, polls until its group's count is complete,
+// invalidates its CU's L1 and requantizes the group's rows straight into its LDS A buffers (the
 // requant kernel's arithmetic, so the same bits; the group's first GEMM2 item also writes act
-// and amax out). Every GEMM1 item is claimed before any GEMM2 item of its XCD, and a GEMM1 item
-// waits on nothing, so every wait ends; a wait is also bounded (kPipeSpinLimit polls), and one
-// that runs out is counted (the launch's last workgroup leaves the count in meta[3], the call's
-// status) instead of hanging. The workgroup that finishes last runs the
-// queue of any XCD that no workgroup ran (none when the launch covers the chip), alone and
-// start to end.
+// and amax out). It reads the rows through its own L2, which holds none of their lines: nothing in
+// this launch reads a row's line before the row's group is complete (a row is whole lines). The
+// maxima, whose lines two groups can share, it reads device-coherent. A workgroup starts on GEMM2
+// items only when every GEMM1 item is claimed, and a GEMM1 item waits on nothing, so every wait
+// ends, also when some XCDs have no workgroups; a wait is also bounded (kPipeSpinLimit polls), and
+// one that runs out is counted (the launch's last workgroup leaves the count in meta[3], the call's
+// status) instead of hanging.
 //
 // Combine (PipeArgs::y set): a GEMM2 item stores its partial rows device-coherent (sc1: written
 // through the XCD's L2, which other XCDs do not see), drains them and counts itself done for its
@@ -1380,9 +1421,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs 
 // routed slot (the task's expert from the routing's LDS table) it waits until the expert's
 // GEMM1 items are done (its rows' output_index entries are written, also device-coherent) and
 // loads the row, then until the expert's GEMM2 items are done, and reads the partial rows with
-// device-coherent loads. Every GEMM2 item is claimed by a workgroup of its XCD, or by the last
-// workgroup for an XCD without any, so every wait ends. The workgroup that leaves last sets the
-// counters back to zero.
+// device-coherent loads. A workgroup starts to combine only when every GEMM2 item is claimed, so
+// every wait ends. The workgroup that leaves last sets the counters back to zero.
 __device__ __forceinline__ int hw_xcc_id() {
   int v;
   asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(v));
@@ -1412,14 +1452,15 @@ __device__ __forceinline__ uint4 ld16_coherent(__amdgpu_buffer_rsrc_t r, int off
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
-// The combine of token t in the decode pipeline (one wave, whole rows of H <= 64 * 8 * 8
-// columns): the slot-ordered fp32 sum of its routed slots' partial rows from +0, bf16 RNE (the
-// combine kernel's arithmetic, so the same bits); a token without routed slots gets zeros.
+// The combine of token t in the decode pipeline (one wave, kPipeCombineV * 512 columns at a time):
+// the slot-ordered fp32 sum of its routed slots' partial rows from +0, bf16 RNE (the combine
+// kernel's arithmetic, so the same bits); a token without routed slots gets zeros.
 constexpr int kPipeCombineV = 8;  // 16-byte column groups per lane
 
 __device__ void pipe_combine_token(const PipeArgs& p, int64_t t, const uint8_t* s_ev,
-                                   const int* s_gprefix, int n1, int n2, const int32_t* done1,
-                                   const int32_t* done2, __amdgpu_buffer_rsrc_t part) {
+                                   const int* s_prefix1, const int* s_prefix2, int n1, int n2,
+                                   const int32_t* done1, const int32_t* done2,
+                                   __amdgpu_buffer_rsrc_t part) {
   constexpr int V = kPipeCombineV;
   const RouteArgs& ra = p.g1.route;
   const int lane = lane_id();
@@ -1431,119 +1472,141 @@ __device__ void pipe_combine_token(const PipeArgs& p, int64_t t, const uint8_t* 
     const int ev = s_ev[task];
     if (ev != 255) {
       bool ok = true;
-      for (int grp = s_gprefix[ev]; grp < s_gprefix[ev + 1]; ++grp)
+      for (int grp = s_prefix1[ev]; grp < s_prefix1[ev + 1]; ++grp)
         ok = ok && wait_count(&done1[grp], n1, p.spin_limit);
       row = __hip_atomic_load(&ra.output_index[task], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      ok = ok && wait_count(&done2[ev * kPipeDone2Stride], n2 * (s_gprefix[ev + 1] - s_gprefix[ev]),
+      ok = ok && wait_count(&done2[ev * kPipeDone2Stride], n2 * (s_prefix2[ev + 1] - s_prefix2[ev]),
                             p.spin_limit);
       if (!ok) atomicAdd(&p.pipe[kPipeFailAt], 1);
     }
   }
-  float sum[V][8];
+  const uint64_t routed = __ballot(row >= 0);
+  uint4* yrow = reinterpret_cast<uint4*>(p.y + t * hidden);
+  for (int v0 = 0; v0 < nvec; v0 += V * kWave) {
+    float sum[V][8];
 #pragma unroll
-  for (int j = 0; j < V; ++j)
+    for (int j = 0; j < V; ++j)
 #pragma unroll
-    for (int q = 0; q < 8; ++q) sum[j][q] = 0.0f;
-  // the routed slots in ascending order, two at a time (their loads go out together)
-  constexpr int kSlots = 2;
-  for (uint64_t m = __ballot(row >= 0); m != 0;) {
-    uint4 pv[kSlots][V];
-    bool has[kSlots];
+      for (int q = 0; q < 8; ++q) sum[j][q] = 0.0f;
+    // the routed slots in ascending order, two at a time (their loads go out together)
+    constexpr int kSlots = 2;
+    for (uint64_t m = routed; m != 0;) {
+      uint4 pv[kSlots][V];
+      bool has[kSlots];
 #pragma unroll
-    for (int b = 0; b < kSlots; ++b) {
-      has[b] = m != 0;  // wave-uniform (a ballot)
-      const int s = has[b] ? __ffsll(static_cast<unsigned long long>(m)) - 1 : 0;
-      m &= m - 1;
-      const int r = __shfl(row, s, kWave);
+      for (int b = 0; b < kSlots; ++b) {
+        has[b] = m != 0;  // wave-uniform (a ballot)
+        const int s = has[b] ? __ffsll(static_cast<unsigned long long>(m)) - 1 : 0;
+        m &= m - 1;
+        const int r = __shfl(row, s, kWave);
 #pragma unroll
-      for (int j = 0; j < V; ++j) {
-        const int v = j * kWave + lane;
-        pv[b][j] = has[b] && v < nvec ? ld16_coherent(part, (r * hidden + v * 8) * 2) : make_uint4(0, 0, 0, 0);
+        for (int j = 0; j < V; ++j) {
+          const int v = v0 + j * kWave + lane;
+          pv[b][j] = has[b] && v < nvec ? ld16_coherent(part, (r * hidden + v * 8) * 2) : make_uint4(0, 0, 0, 0);
+        }
       }
-    }
 #pragma unroll
-    for (int b = 0; b < kSlots; ++b) {
-      if (!has[b]) break;
+      for (int b = 0; b < kSlots; ++b) {
+        if (!has[b]) break;
 #pragma unroll
-      for (int j = 0; j < V; ++j) {
-        const uint32_t words[4] = {pv[b][j].x, pv[b][j].y, pv[b][j].z, pv[b][j].w};
+        for (int j = 0; j < V; ++j) {
+          const uint32_t words[4] = {pv[b][j].x, pv[b][j].y, pv[b][j].z, pv[b][j].w};
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          sum[j][2 * q] += bf16_to_f32(words[q] & 0xffff);
-          sum[j][2 * q + 1] += bf16_to_f32(words[q] >> 16);
+          for (int q = 0; q < 4; ++q) {
+            sum[j][2 * q] += bf16_to_f32(words[q] & 0xffff);
+            sum[j][2 * q + 1] += bf16_to_f32(words[q] >> 16);
+          }
         }
       }
     }
-  }
-  uint4* yrow = reinterpret_cast<uint4*>(p.y + t * hidden);
 #pragma unroll
-  for (int j = 0; j < V; ++j) {
-    const int v = j * kWave + lane;
-    if (v < nvec)
-      yrow[v] = make_uint4(pack_bf16x2(sum[j][0], sum[j][1]), pack_bf16x2(sum[j][2], sum[j][3]),
-                           pack_bf16x2(sum[j][4], sum[j][5]), pack_bf16x2(sum[j][6], sum[j][7]));
+    for (int j = 0; j < V; ++j) {
+      const int v = v0 + j * kWave + lane;
+      if (v < nvec)
+        yrow[v] = make_uint4(pack_bf16x2(sum[j][0], sum[j][1]), pack_bf16x2(sum[j][2], sum[j][3]),
+                             pack_bf16x2(sum[j][4], sum[j][5]), pack_bf16x2(sum[j][6], sum[j][7]));
+    }
   }
 }
 
-// Wave 0: s_gprefix[0..E] = exclusive prefix of the experts' groups (chunks of kStreamRows rows).
-__device__ void plan_groups(int E, const int* s_count, int* s_gprefix) {
+// The two kernels of the pipeline: for few tasks (kPipeSmallTasks) chunks of up to 32 rows and items
+// of 2, 4 or 8 units, else chunks of up to 128 rows in GEMM1 and of 64 rows in GEMM2 (whose A rows
+// are resident in LDS) and whole items.
+//
+// 64-column units (waves) of an item of the small kernel when there are G groups: the widest items
+// that still give most CUs one. A CU reads at most ~50 GB/s, so ~140 of them saturate the HBM, and
+// whole items (8 waves) do that from 17 groups on; with fewer groups the same columns go to more CUs
+// in narrower items. At least 2: the 64 channels that two units of GEMM1 write to a row of y are one
+// 128-byte line, which then comes from one workgroup. 6 rows on 6 experts (4096 x 4096 and 4096 x
+// 2048): 66 us with 48 of the 256 CUs on whole items, 34 us with items of 2 units on 192.
+template <bool kSmall>
+struct PipeShape {
+  static constexpr int kRows1 = kSmall ? 32 : kStreamItemRows;  // rows of a GEMM1 item (a group)
+  static constexpr int kRows2 = kSmall ? 32 : kStreamRows;      // rows of a GEMM2 item
+  static_assert(kRows1 % kRows2 == 0, "a GEMM2 item's rows are one group's");
+  static __device__ __forceinline__ int units(int G) { return !kSmall || G > 16 ? kGemmWaves : G > 8 ? 4 : 2; }
+};
+
+// Wave 0: s_prefix[0..E] = exclusive prefix of the experts' chunks of `rows` rows; their number.
+__device__ int plan_chunks(int E, int rows, const int* s_count, int* s_prefix) {
   const int lane = lane_id();
   int carry = 0;
   for (int e0 = 0; e0 < E; e0 += kWave) {
     const int e = e0 + lane;
-    const int n = e < E ? (s_count[e] + kStreamRows - 1) / kStreamRows : 0;
+    const int n = e < E ? (s_count[e] + rows - 1) / rows : 0;
     const int inc = wave_inclusive_sum(n);
-    if (e < E) s_gprefix[e] = carry + inc - n;
+    if (e < E) s_prefix[e] = carry + inc - n;
     carry += __shfl(inc, kWave - 1, kWave);
   }
-  if (lane == 0) s_gprefix[E] = carry;
+  if (lane == 0) s_prefix[E] = carry;
+  return carry;
 }
 
 // The requant of rows [row0, row0 + mrows) of GEMM1's bf16 output y into the LDS A chunk buffers
-// of a STREAM GEMM2 tile of MT 32-row tiles (stream_tile's chunk layout; K = I in one chunk for
-// MT = 1, two for MT = 2): the row's amax, inv = 448 / max(amax, 1e-4), then 16 e4m3 codes per
+// of a STREAM GEMM2 tile of MT 32-row tiles (stream_tile's chunk layout; K = I in at most two chunks
+// of kc): the row's amax, inv = 448 / max(amax, 1e-4), then 16 e4m3 codes per
 // LDS piece -- the requant kernel's arithmetic, so the same bits. The amax is the max of the
-// row's 64 partial maxima that GEMM1's epilogue stored (one per 64-column block, exact), eight
+// row's 2I/64 partial maxima that GEMM1's epilogue stored (one per 64-column block, exact), eight
 // lanes a row. The row scale a/448 goes straight into the tile's LDS scale table (s_xs); with
 // write_act the rows' act, act_scale and amax also go out. The y pieces go out kStageBatch at a
 // time, the first batch together with the maxima; rows past mrows are neither loaded nor
 // quantized (their LDS rows feed only accumulator rows that are never stored).
-constexpr int kStageBatch = 4;
+constexpr int kPipeMaxInter = 2 * kAChunk / kStreamRows;  // I of a group's rows in both A buffers
 
-template <int MT>
-__device__ void stage_rows_from_y(const PipeArgs& p, int row0, int mrows, bool write_act,
+template <int MT, int kStageBatch>
+__device__ void stage_rows_from_y(const PipeArgs& p, int row0, int mrows, int kc, bool write_act,
                                   uint8_t* smem, float* s_inv, float* s_xs) {
-  constexpr int kc = kAChunk / (32 * MT);
-  constexpr int kUnits = 2 * 2048 / kStreamUnit;  // partial maxima per row (I = 2048)
+  using Chunk = AChunk<MT>;
+  constexpr int kUnitsPerLane = 2 * kPipeMaxInter / kStreamUnit / 8;
   static_assert(kStreamRows == kGemmWaves * kWave / 8, "eight lanes per row cover the group");
   static_assert(kALoads % kStageBatch == 0, "whole batches");
   const int inter = p.g1.sw.inter;
+  const int units = 2 * inter / kStreamUnit;
   const int nchunks = inter / kc;
   const int tid = opaque_tid();
   const int lane = tid & (kWave - 1), wave = tid / kWave;
   const uint16_t* y = p.g1.sw.y;
   const int r8 = tid >> 3;
-  float4 pm[kUnits / 32];
+  float pm[kUnitsPerLane];
 #pragma unroll
-  for (int j = 0; j < kUnits / 32; ++j) pm[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  if (r8 < mrows) {
-    const float4* src = reinterpret_cast<const float4*>(
-        p.g1.row_pmax + static_cast<int64_t>(row0 + r8) * kUnits + (tid & 7) * (kUnits / 8));
-#pragma unroll
-    for (int j = 0; j < kUnits / 32; ++j) pm[j] = src[j];
+  for (int j = 0; j < kUnitsPerLane; ++j) {
+    const int u = j * 8 + (tid & 7);
+    pm[j] = 0.0f;
+    if (r8 < mrows && u < units)
+      pm[j] = __hip_atomic_load(p.g1.row_pmax + static_cast<int64_t>(row0 + r8) * units + u, __ATOMIC_RELAXED,
+                                __HIP_MEMORY_SCOPE_AGENT);
   }
-  // batch b of chunk c: pieces i = b * kStageBatch + h; piece i of a lane holds LDS bytes
-  // (i * 8 + wave) * 1024 + lane * 16 of the chunk buffer (row r, swizzled piece): 16 channels,
-  // 32 bytes of y
+  // batch b of chunk c: pieces i = b * kStageBatch + h of the chunk: 16 channels, 32 bytes of y
   uint4 v[kStageBatch][2];
+  auto valid = [&](int i) { return Chunk::row(i, lane, wave) < mrows; };
+  auto source = [&](int c, int i) { return c * kc + Chunk::src(i, lane, wave, kc) * 16; };  // piece i's channel
   auto load_batch = [&](int c, int b) {
 #pragma unroll
     for (int h = 0; h < kStageBatch; ++h) {
-      const int pos = ((b * kStageBatch + h) * kGemmWaves + wave) * 1024 + lane * 16;
-      const int r = pos / kc;
-      const int off = c * kc + swizzle_piece((pos - r * kc) >> 4, r) * 16;
-      if (r < mrows) {
-        const uint4* src = reinterpret_cast<const uint4*>(y + static_cast<int64_t>(row0 + r) * inter + off);
+      const int i = b * kStageBatch + h;
+      if (valid(i)) {
+        const uint4* src = reinterpret_cast<const uint4*>(
+            y + static_cast<int64_t>(row0 + Chunk::row(i, lane, wave)) * inter + source(c, i));
         v[h][0] = src[0];
         v[h][1] = src[1];
       }
@@ -1555,7 +1618,7 @@ __device__ void stage_rows_from_y(const PipeArgs& p, int row0, int mrows, bool w
   {
     float m = 0.0f;
 #pragma unroll
-    for (int j = 0; j < kUnits / 32; ++j) m = fmaxf(fmaxf(fmaxf(m, pm[j].x), fmaxf(pm[j].y, pm[j].z)), pm[j].w);
+    for (int j = 0; j < kUnitsPerLane; ++j) m = fmaxf(m, pm[j]);
 #pragma unroll
     for (int off = 1; off < 8; off <<= 1) m = fmaxf(m, __shfl_xor(m, off, kWave));
     if ((tid & 7) == 0 && r8 < mrows) {
@@ -1574,30 +1637,65 @@ __device__ void stage_rows_from_y(const PipeArgs& p, int row0, int mrows, bool w
 #pragma unroll
       for (int h = 0; h < kStageBatch; ++h) {
         const int i = b * kStageBatch + h;
-        const int pos = (i * kGemmWaves + wave) * 1024 + lane * 16;
-        const int r = pos / kc;
+        const int r = Chunk::row(i, lane, wave);
         int4 q = make_int4(0, 0, 0, 0);  // rows past mrows: never stored
-        if (r < mrows) {
+        if (valid(i)) {
           const float inv = s_inv[r];
           const uint4 a = v[h][0], b2 = v[h][1];
           q.x = static_cast<int>(pack_e4m3x4(lo(a.x) * inv, hi(a.x) * inv, lo(a.y) * inv, hi(a.y) * inv));
           q.y = static_cast<int>(pack_e4m3x4(lo(a.z) * inv, hi(a.z) * inv, lo(a.w) * inv, hi(a.w) * inv));
           q.z = static_cast<int>(pack_e4m3x4(lo(b2.x) * inv, hi(b2.x) * inv, lo(b2.y) * inv, hi(b2.y) * inv));
           q.w = static_cast<int>(pack_e4m3x4(lo(b2.z) * inv, hi(b2.z) * inv, lo(b2.w) * inv, hi(b2.w) * inv));
-          if (write_act) {
-            const int off = c * kc + swizzle_piece((pos - r * kc) >> 4, r) * 16;
-            *reinterpret_cast<int4*>(p.act + static_cast<int64_t>(row0 + r) * inter + off) = q;
-          }
+          if (write_act)
+            *reinterpret_cast<int4*>(p.act + static_cast<int64_t>(row0 + r) * inter + source(c, i)) = q;
         }
-        *reinterpret_cast<int4*>(smem + (c & 1) * kAChunk + wave * 1024 + lane * 16 + i * kGemmWaves * 1024) = q;
+        *reinterpret_cast<int4*>(smem + (c & 1) * kAChunk + r * Chunk::kMaxK + Chunk::pos(i, lane) * 16) = q;
       }
     }
   }
 }
 
+// The items [0, total) of one GEMM dealt to the XCDs in equal contiguous ranges. Wave 0 holds in one
+// register (`held`) the workgroup's next claim (lane 0) and what the XCDs' counters read when that
+// claim went out (XCD q's in lane kPeekLane + q).
+constexpr int kPeekLane = 8;
+struct PipeDeal {
+  int32_t* claims;  // XCD x's counter at claims[x * kPipeLine]
+  int total;
+  __device__ __forceinline__ int begin(int x) const { return static_cast<int>(static_cast<int64_t>(total) * x / kPipeXcds); }
+  __device__ __forceinline__ int size(int x) const { return begin(x + 1) - begin(x); }
+  // wave 0: claims the next item of XCD x and peeks at all counters
+  __device__ __forceinline__ int claim(int x) const {
+    const int lane = lane_id();
+    int held = 0;
+    if (lane == 0) held = atomicAdd(&claims[x * kPipeLine], 1);
+    else if (lane >= kPeekLane && lane < kPeekLane + kPipeXcds)
+      held = __hip_atomic_load(&claims[(lane - kPeekLane) * kPipeLine], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return held;
+  }
+  // wave 0: the XCDs with items left by a peek (claims only grow: an empty mask stays empty)
+  __device__ __forceinline__ uint32_t left(int held) const {
+    const int q = lane_id() - kPeekLane;
+    return static_cast<uint32_t>(__ballot(q >= 0 && q < kPipeXcds && held < size(q & (kPipeXcds - 1))) >> kPeekLane);
+  }
+};
+
+// The kernel's argument block through a pointer that is opaque to the optimizer, one for each item:
+// what an item needs of the 900 bytes is then read (from the scalar cache) in that item. Read
+// through the argument itself, all of it was hoisted in front of the item loop and spilled there
+// (180 scalar registers).
+__device__ __forceinline__ const PipeArgs& item_args() {
+  uint64_t at = reinterpret_cast<uint64_t>(__builtin_amdgcn_kernarg_segment_ptr());
+  asm volatile("" : "+s"(at));
+  return *(const PipeArgs*)(const __attribute__((address_space(4))) PipeArgs*)(at);
+}
+
+template <bool kSmall>
 __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeArgs p) {
+  using Shape = PipeShape<kSmall>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  __shared__ int s_gprefix[kMaxGemmExperts + 1];
+  __shared__ int s_prefix1[kMaxGemmExperts + 1];  // the experts' chunks: GEMM1 (groups), GEMM2
+  __shared__ int s_prefix2[kMaxGemmExperts + 1];
   __shared__ int s_count[kMaxGemmExperts];
   __shared__ int s_off[kMaxGemmExperts + 1];
   __shared__ int s_wcnt[kGemmWaves][kMaxGemmExperts];
@@ -1607,32 +1705,45 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
   __shared__ uint8_t s_ev[kFusedMaxTasks];
   __shared__ TileTables s_tt;
   __shared__ float s_inv[kStreamRows];
-  __shared__ int s_word;  // thread 0 -> the workgroup
+  __shared__ int s_word;    // wave 0 -> the workgroup
+  __shared__ int s_claim2;  // the first GEMM2 claim
+  __shared__ int s_rows1;   // rows of a group
   const GemmArgs& g1 = p.g1;
   const GemmArgs& g2 = p.g2;
   const RouteArgs& ra = g1.route;
   const int E = g1.num_experts;
-  int32_t* const claims = p.pipe;  // XCD x's counter at claims[x * kPipeLine]
-  int32_t* const finish = p.pipe + kPipeFinishAt;
   int32_t* const done1 = p.pipe + kPipeDone1At;  // [groups]
   int32_t* const done2 = p.pipe + kPipeDone2At;  // [experts]
-  const int hw = hw_xcc_id();
-  const int home = hw & (kPipeXcds - 1);
-  int x = home;
-  // thread 0: the first claim (its latency hides behind the routing); a workgroup's home XCD
-  // counter is nonzero from then on, which is how the last workgroup finds XCDs without any
-  int pending = 0;
-  if (threadIdx.x == 0) pending = atomicAdd(&claims[x * kPipeLine], 1);
+  const int home = hw_xcc_id() & (kPipeXcds - 1);
+  // wave 0: the first claims of both GEMMs (their latency hides behind the routing; nothing is known
+  // to be left then, and a peek of zeros says nothing)
+  int held = 0, held2 = 0;
+  if (threadIdx.x == 0) {
+    held = atomicAdd(&p.pipe[home * kPipeLine], 1);
+    held2 = atomicAdd(&p.pipe[home * kPipeLine + kPipeClaim2], 1);
+  }
   const int ntasks = effective_tokens(ra.runtime_tokens, ra.host_tokens) * ra.topk;
   {
     const int wave = static_cast<int>(threadIdx.x) / kWave;
     for (int e = lane_id(); e < E; e += kWave) s_wcnt[wave][e] = 0;
   }
   fused_count(ra, ntasks, s_wcnt, s_ev, reinterpret_cast<float*>(smem), blockIdx.x == 0);
+  if (threadIdx.x == 0) s_claim2 = held2;
   __syncthreads();
   if (threadIdx.x < kWave) {
     fused_scan(E, s_wcnt, s_count, s_off);
-    plan_groups(E, s_count, s_gprefix);
+    // groups of GEMM2's rows when they take no more rounds of items than the larger ones: an item of 4
+    // row tiles has half the weight steps in flight (2046 Zipf rows: 217 us in 128-row groups, 199
+    // in 64-row ones, both two rounds; 3072 even rows, one round against two: 203 and 223)
+    const int n = stream_blocks(g1), cus = static_cast<int>(gridDim.x);
+    int rows = Shape::kRows1;
+    const int chunks1 = plan_chunks(E, rows, s_count, s_prefix1);
+    const int chunks2 = plan_chunks(E, Shape::kRows2, s_count, s_prefix2);
+    if (Shape::kRows1 != Shape::kRows2 && (chunks2 * n + cus - 1) / cus <= (chunks1 * n + cus - 1) / cus) {
+      rows = Shape::kRows2;
+      plan_chunks(E, rows, s_count, s_prefix1);
+    }
+    if (threadIdx.x == 0) s_rows1 = rows;
   }
   __syncthreads();
   if (blockIdx.x == 0) {  // the routing outputs that the later stages read
@@ -1645,98 +1756,111 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
       ra.meta[0] = s_off[E] < ra.row_cap ? s_off[E] : static_cast<int>(ra.row_cap);
       p.meta[1] = 0;  // the 8-wave GEMM1
       if (p.direct_flag != nullptr) *p.direct_flag = 0;
-      if (hw >= kPipeXcds) atomicAdd(&p.pipe[kPipeFailAt], 1);  // an XCD id this launch does not expect
     }
   }
   // more groups than counters (the host's task bound rules it out): flagged, and no items
-  const bool too_many = s_gprefix[E] > kMaxPipeGroups;
+  const bool too_many = s_prefix1[E] > kMaxPipeGroups;
   if (too_many && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&p.pipe[kPipeFailAt], 1);
-  const int G = too_many ? 0 : s_gprefix[E];
-  const int n1 = stream_blocks(g1), n2 = stream_blocks(g2);
+  const int G = __builtin_amdgcn_readfirstlane(too_many ? 0 : s_prefix1[E]);
+  const int waves = Shape::units(G);
+  const int n1 = g1.n / (kStreamUnit * waves), n2 = g2.n / (kStreamUnit * waves);
   const float* task_w = reinterpret_cast<const float*>(smem);  // valid until the first item's loads
   bool first_item = true;
-  int present = -1;  // the last workgroup: XCDs that had workgroups (bit mask)
-  int orphan = -1;   // the last workgroup: the XCD queue it runs
-  for (;;) {
-    if (threadIdx.x == 0) s_word = pending;
-    __syncthreads();
-    const int t = s_word;
-    __syncthreads();
-    const int gb = static_cast<int>(static_cast<int64_t>(G) * x / kPipeXcds);
-    const int ng = static_cast<int>(static_cast<int64_t>(G) * (x + 1) / kPipeXcds) - gb;
-    if (t >= (n1 + n2) * ng) {
-      if (present < 0) {
-        // count this workgroup finished (after its last claim was answered); the last one
-        // learns which XCDs had workgroups: those whose claim counter moved
-        if (threadIdx.x == 0) {
-          const bool is_last = atomicAdd(finish, 1) == static_cast<int>(gridDim.x) - 1;
-          int mask = -1;
-          if (is_last) {
-            mask = 0;
-            for (int q = 0; q < kPipeXcds; ++q)
-              if (__hip_atomic_load(&claims[q * kPipeLine], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
-                mask |= 1 << q;
+  for (int phase = 0; phase < 2; ++phase) {
+    const bool gemm1 = phase == 0;
+    const PipeDeal deal{p.pipe + (gemm1 ? 0 : kPipeClaim2),
+                        gemm1 ? G * n1 : too_many ? 0 : __builtin_amdgcn_readfirstlane(s_prefix2[E]) * n2};
+    if (!gemm1) held = threadIdx.x == 0 ? s_claim2 : 0;
+    int x = home;
+    for (;;) {
+      if (threadIdx.x == 0) s_word = held;
+      __syncthreads();
+      const int c = __builtin_amdgcn_readfirstlane(s_word);
+      __syncthreads();
+      if (c >= deal.size(x)) {
+        // this range is claimed: an XCD with items left, the next one from here on, or the next phase
+        if (threadIdx.x < kWave) {
+          uint32_t left = deal.left(held);
+          while (left != 0) {  // (each round claims an item, or finds one range more claimed out)
+            const uint32_t turned = (left | left << kPipeXcds) >> home;
+            x = (home + __ffs(static_cast<int>(turned)) - 1) & (kPipeXcds - 1);
+            held = deal.claim(x);
+            if (__shfl(held, 0, kWave) < deal.size(x)) break;
+            left = deal.left(held) & ~(1u << x);
           }
-          s_word = mask;
+          if (threadIdx.x == 0) s_word = left == 0 ? -1 : x;
         }
         __syncthreads();
-        present = s_word;
+        x = __builtin_amdgcn_readfirstlane(s_word);
         __syncthreads();
-        if (present < 0) break;
+        if (x < 0) break;
+        continue;
       }
-      // every other workgroup has finished: the queues of XCDs without workgroups, whole
-      do ++orphan; while (orphan < kPipeXcds && ((present >> orphan) & 1));
-      if (orphan >= kPipeXcds) break;
-      x = orphan;
-      if (threadIdx.x == 0) pending = atomicAdd(&claims[x * kPipeLine], 1);
-      continue;
-    }
-    if (threadIdx.x == 0) pending = atomicAdd(&claims[x * kPipeLine], 1);  // the next claim, one item ahead
-    const bool gemm1 = t < n1 * ng;
-    const int local = gemm1 ? t : t - n1 * ng;
-    const int per = gemm1 ? n1 : n2;
-    const int grp = gb + local / per;
-    const int nb = local - (local / per) * per;
-    const int e = expert_of_item(s_gprefix, E, grp);
-    const int r0 = (grp - s_gprefix[e]) * kStreamRows;
-    const int cnt = s_count[e];
-    const int off_e = s_off[e];
-    const int mrows = min(kStreamRows, cnt - r0);
-    const int row0 = off_e + r0;
-    if (gemm1) {
-      // the weights go out first; then the item's rows are ranked into the LDS row table
-      const float* item_w = first_item ? task_w : nullptr;
-      const auto rank_rows = [&]() {
-        fused_rows(ra, ntasks, e, cnt, off_e, s_wcnt, s_ev, item_w, r0, nb == 0 ? r0 : 0,
-                   nb == 0 ? r0 + kStreamRows : 0, 0, 0, s_task, s_tok, s_rw);
-      };
-      const RowSrc rs{s_tok, s_rw, row0};
-      if (mrows > 32) stream_tile<true, true, 2, true, true, false, true, true>(g1, rs, e, row0, mrows, nb, smem, s_tt, rank_rows);
-      else stream_tile<true, true, 1, true, true, false, true, true>(g1, rs, e, row0, mrows, nb, smem, s_tt, rank_rows);
-      vm_drain();  // this wave's y stores are in L2
-      __syncthreads();
-      if (threadIdx.x == 0) atomicAdd(&done1[grp], 1);
-    } else {
-      // the weights go out first; then the group's rows, requantized from y into LDS
-      const auto stage_rows = [&]() {
-        if (threadIdx.x == 0 && !wait_count(&done1[grp], n1, p.spin_limit)) atomicAdd(&p.pipe[kPipeFailAt], 1);
+      if (threadIdx.x < kWave) held = deal.claim(x);  // the next claim, one item ahead
+      const PipeArgs& q = item_args();
+      // item t: an expert's items column block by column block, the chunks of a block next to each
+      // other, so that they run together and read its weights from HBM once
+      const int t = deal.begin(x) + c;
+      const int* s_prefix = gemm1 ? s_prefix1 : s_prefix2;
+      const int per = gemm1 ? n1 : n2;
+      const int e = expert_of_item(s_prefix, E, t / per);
+      const int first = __builtin_amdgcn_readfirstlane(s_prefix[e]);
+      const int nch = __builtin_amdgcn_readfirstlane(s_prefix[e + 1]) - first;
+      const int nb = (t - first * per) / nch;
+      const int ch = t - first * per - nb * nch;
+      const int rows1 = __builtin_amdgcn_readfirstlane(s_rows1);
+      const int rows = gemm1 ? rows1 : Shape::kRows2;
+      const int r0 = ch * rows;
+      const int cnt = __builtin_amdgcn_readfirstlane(s_count[e]);
+      const int off_e = __builtin_amdgcn_readfirstlane(s_off[e]);
+      const int mrows = min(rows, cnt - r0);
+      const int row0 = off_e + r0;
+      const int grp = gemm1 ? first + ch : __builtin_amdgcn_readfirstlane(s_prefix1[e]) + r0 / rows1;
+      if (gemm1) {
+        // the weights go out first; then the item's rows are ranked into the LDS row table
+        const float* item_w = first_item ? task_w : nullptr;
+        const auto rank_rows = [&]() {
+          fused_rows(q.g1.route, ntasks, e, cnt, off_e, s_wcnt, s_ev, item_w, r0, nb == 0 ? r0 : 0,
+                     nb == 0 ? r0 + rows1 : 0, 0, 0, s_task, s_tok, s_rw);
+        };
+        const RowSrc rs{s_tok, s_rw, row0};
+        if (kSmall && waves < kGemmWaves)
+          stream_tile<true, true, 1, kNarrowDepth, true, false, true, true, true, kALoads / 2>(q.g1, rs, e, row0, mrows, nb, q.narrow_kc1, smem, s_tt, rank_rows, waves);
+        else if (!kSmall && mrows > 64)
+          stream_tile<true, true, 4, 2, true, false, true, true, false, kALoads / 2>(q.g1, rs, e, row0, mrows, nb, q.half_kc4, smem, s_tt, rank_rows);
+        else if (!kSmall && mrows > 32)
+          stream_tile<true, true, 2, kStreamDepth, true, false, true, true>(q.g1, rs, e, row0, mrows, nb, q.g1.kc[1], smem, s_tt, rank_rows);
+        else
+          stream_tile<true, true, 1, kStreamDepth, true, false, true, true>(q.g1, rs, e, row0, mrows, nb, q.g1.kc[0], smem, s_tt, rank_rows);
+        vm_drain();  // this wave's y stores are written through to the device-coherent level
         __syncthreads();
-        l1_invalidate();
-        if (mrows > 32) stage_rows_from_y<2>(p, row0, mrows, nb == 0, smem, s_inv, s_tt.xs);
-        else stage_rows_from_y<1>(p, row0, mrows, nb == 0, smem, s_inv, s_tt.xs);
+        if (threadIdx.x == 0) atomicAdd(&q.pipe[kPipeDone1At + grp], 1);
+      } else {
+        // the weights go out first; then the group's rows, requantized from y into LDS
+        const auto stage_rows = [&]() {
+          if (threadIdx.x == 0 && !wait_count(&q.pipe[kPipeDone1At + grp], n1, q.spin_limit)) atomicAdd(&q.pipe[kPipeFailAt], 1);
+          __syncthreads();
+          l1_invalidate();
+          // (beside a ring of 8 steps there are registers for two pieces at a time)
+          if constexpr (kSmall) stage_rows_from_y<1, 2>(q, row0, mrows, q.g2.kc[0], nb == 0, smem, s_inv, s_tt.xs);
+          else if (mrows > 32) stage_rows_from_y<2, 4>(q, row0, mrows, q.g2.kc[1], nb == 0, smem, s_inv, s_tt.xs);
+          else stage_rows_from_y<1, 4>(q, row0, mrows, q.g2.kc[0], nb == 0, smem, s_inv, s_tt.xs);
+          __syncthreads();
+        };
+        const RowSrc rs{nullptr, nullptr, 0};
+        if (kSmall && waves < kGemmWaves)
+          stream_tile<false, false, 1, kNarrowDepth, true, true, false, true, true>(q.g2, rs, e, row0, mrows, nb, q.g2.kc[0], smem, s_tt, stage_rows, waves);
+        else if (!kSmall && mrows > 32)
+          stream_tile<false, false, 2, kStreamDepth, true, true, false, true>(q.g2, rs, e, row0, mrows, nb, q.g2.kc[1], smem, s_tt, stage_rows);
+        else
+          stream_tile<false, false, 1, kStreamDepth, true, true, false, true>(q.g2, rs, e, row0, mrows, nb, q.g2.kc[0], smem, s_tt, stage_rows);
+        vm_drain();  // this wave's partial rows are written through to the device-coherent level
         __syncthreads();
-      };
-      const RowSrc rs{nullptr, nullptr, 0};
-      if (mrows > 32)
-        stream_tile<false, false, 2, true, true, true, false, true>(g2, rs, e, row0, mrows, nb, smem, s_tt, stage_rows);
-      else
-        stream_tile<false, false, 1, true, true, true, false, true>(g2, rs, e, row0, mrows, nb, smem, s_tt, stage_rows);
-      vm_drain();  // this wave's partial rows are written through to the device-coherent level
+        if (threadIdx.x == 0) atomicAdd(&q.pipe[kPipeDone2At + e * kPipeDone2Stride], 1);
+      }
+      first_item = false;
       __syncthreads();
-      if (threadIdx.x == 0) atomicAdd(&done2[e * kPipeDone2Stride], 1);
     }
-    first_item = false;
-    __syncthreads();
   }
   if (p.y != nullptr && !too_many) {
     // the combine: token i goes to wave (i / gridDim.x) % 8 of workgroup i % gridDim.x, so the
@@ -1748,7 +1872,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
     const int wave = static_cast<int>(threadIdx.x) / kWave;
     for (int64_t t = blockIdx.x + static_cast<int64_t>(wave) * gridDim.x; t < tokens;
          t += static_cast<int64_t>(gridDim.x) * kGemmWaves)
-      pipe_combine_token(p, t, s_ev, s_gprefix, n1, n2, done1, done2, part);
+      pipe_combine_token(p, t, s_ev, s_prefix1, s_prefix2, n1, n2, done1, done2, part);
   }
   // the workgroup that leaves last (every other one has made its last counter access): the
   // count of waits that ran out into meta[3] (the call's status), the counters back to zero
@@ -1945,10 +2069,33 @@ hipError_t launch_engines_k(const GemmArgs& g, int max_rows, int num_cus, hipStr
                        dim3(kGemmThreads), kSmemBytes, stream, g);
 }
 
+// The largest multiple of 64 * steps that divides k and is at most cap; 0: there is none.
+int stream_chunk(int k, int cap, int steps) {
+  for (int kc = cap / (64 * steps) * (64 * steps); kc > 0; kc -= 64 * steps)
+    if (k % kc == 0) return kc;
+  return 0;
+}
+
+// The STREAM engine's chunks of K for 1, 2 and 4 row tiles: as long as the LDS buffers allow, so that
+// the workgroup's barriers are few, with a ring of 4 weight steps unless a ring of 2 makes a chunk at
+// least twice as long (K not a multiple of 256: 640 = 10 steps). Four row tiles always have 2.
+void set_stream_chunks(GemmArgs* g) {
+  for (int i = 0; i < 3; ++i) {
+    const int cap = kAChunk / 32 >> i;
+    const int four = i < 2 ? stream_chunk(g->k, cap, kStreamDepth) : 0;
+    const int two = stream_chunk(g->k, cap, 2);
+    g->ring[i] = 2 * four > two ? kStreamDepth : 2;
+    g->kc[i] = 2 * four > two ? four : two;
+  }
+}
+
 template <bool kGather, bool kSwiglu>
-hipError_t launch_engines(const GemmArgs& g, int max_rows, int num_cus, hipStream_t stream) {
-  return g.k % (kAChunk / 32) == 0 ? launch_engines_k<kGather, kSwiglu, false>(g, max_rows, num_cus, stream)
-                                    : launch_engines_k<kGather, kSwiglu, true>(g, max_rows, num_cus, stream);
+hipError_t launch_engines(const GemmArgs& args, int max_rows, int num_cus, hipStream_t stream) {
+  GemmArgs g = args;
+  set_stream_chunks(&g);
+  return g.ring[0] == 4 && g.ring[1] == 4
+             ? launch_engines_k<kGather, kSwiglu, false>(g, max_rows, num_cus, stream)
+             : launch_engines_k<kGather, kSwiglu, true>(g, max_rows, num_cus, stream);
 }
 
 }  // namespace
@@ -1998,27 +2145,54 @@ bool gemm_eager_dual(const GemmArgs& g, int max_rows) {
          static_cast<int64_t>(max_rows) < 8ll * kStreamAutoMaxRows * g.num_experts;
 }
 
-// The decode pipeline needs the streaming engine's full-chunk shapes for both GEMMs (GEMM2's
-// K = I in at most two chunks, staged whole by the requant), GEMM1's in-kernel routing, and
-// the whole MI355X (8 XCDs of 32 CUs: its queues are the hardware XCD ids).
+// Tasks (S * K) up to which the pipeline's small kernel runs. At 4096 x 4096 and 4096 x 2048, top-6,
+// 32 of 256 experts local: 34 against 70 us on the large one at 8 tokens, 56 / 77 at 24, 90 / 96 at
+// 48; from ~22 experts with rows on they tie (64 tokens: 105 both). A chunk is 32 rows here, so a
+// skewed load past this bound pays for it: 80 tokens on 26 of 28 Zipf experts 178 against 135 us.
+constexpr int kPipeSmallTasks = 320;
+
+static bool pipe_small(const GemmArgs& g1) {
+  return static_cast<int64_t>(g1.route.host_tokens) * g1.route.topk <= kPipeSmallTasks;
+}
+
+// The decode pipeline needs rings of 4 weight steps and whole items for both GEMMs, GEMM2's K = I
+// in at most two chunks (staged whole by the requant) of an even number of narrow rings, GEMM1's
+// in-kernel routing, and the whole MI355X (8 XCDs of 32 CUs: its queues are the hardware XCD ids).
+// Past the small kernel's tasks it also wants whole A chunks in both GEMMs: at H = 7168 or I = 1536
+// the separate launches are as fast there with few rows an expert (I = 1536, 512 tokens of 128
+// experts: 120 us against 116) and faster with many (R = 2139: 204 against 130).
 bool decode_pipeline_supported(const GemmArgs& g1, const GemmArgs& g2, int num_cus) {
+  GemmArgs c1 = g1, c2 = g2;
+  set_stream_chunks(&c1);
+  set_stream_chunks(&c2);
+  const bool whole_chunks = g1.k % (kAChunk / 32) == 0 && g2.k == kAChunk / 32;
   return num_cus == kPipeXcds * 32 && g1.engine != GemmEngine::kTile && g2.engine != GemmEngine::kTile &&
          g1.route_in_kernel == 1 && g1.sw.enabled && g1.num_experts <= kFusedMaxExperts &&
-         g1.k % (kAChunk / 32) == 0 && g2.k == kAChunk / 32 && g1.n == 2 * g1.sw.inter &&
-         g2.k == g1.sw.inter && g1.n % (kStreamUnit * kGemmWaves) == 0 &&
+         (whole_chunks || pipe_small(g1)) &&
+         c1.ring[0] == kStreamDepth && c1.ring[1] == kStreamDepth && c2.ring[0] == kStreamDepth &&
+         c2.ring[1] == kStreamDepth && stream_chunk(g1.k, kAChunk / 64, kNarrowDepth) > 0 &&
+         g2.k <= kPipeMaxInter && c2.kc[0] == g2.k && 2 * c2.kc[1] >= g2.k && g2.k % (64 * kNarrowDepth) == 0 &&
+         g1.n == 2 * g1.sw.inter && g2.k == g1.sw.inter && g1.n % (kStreamUnit * kGemmWaves) == 0 &&
          g2.n % (kStreamUnit * kGemmWaves) == 0 && g1.row_token != nullptr && g2.row_token == nullptr &&
          g1.dual_rows == nullptr && g2.dual_rows == nullptr && g2.y_direct == nullptr;
 }
 
-hipError_t launch_decode_pipeline(const PipeArgs& p, int num_cus, hipStream_t stream) {
-  if (!decode_pipeline_supported(p.g1, p.g2, num_cus) || p.pipe == nullptr || p.g1.row_pmax == nullptr ||
-      p.act != p.g2.a ||
-      p.act_scale != p.g2.a_scale || p.g2.lda != p.g1.sw.inter)
+hipError_t launch_decode_pipeline(const PipeArgs& args, int num_cus, hipStream_t stream) {
+  if (!decode_pipeline_supported(args.g1, args.g2, num_cus) || args.pipe == nullptr ||
+      args.g1.row_pmax == nullptr || args.act != args.g2.a || args.act_scale != args.g2.a_scale ||
+      args.g2.lda != args.g1.sw.inter)
     return hipErrorInvalidValue;
-  const hipError_t err = ensure_dynamic_lds<&decode_pipeline_kernel>(kSmemBytes);
+  const bool small = pipe_small(args.g1);
+  const hipError_t err = small ? ensure_dynamic_lds<&decode_pipeline_kernel<true>>(kSmemBytes)
+                               : ensure_dynamic_lds<&decode_pipeline_kernel<false>>(kSmemBytes);
   if (err != hipSuccess) return err;
-  return launch_kernel(decode_pipeline_kernel, dim3(static_cast<unsigned>(num_cus)), dim3(kGemmThreads),
-                       kSmemBytes, stream, p);
+  PipeArgs p = args;
+  set_stream_chunks(&p.g1);
+  set_stream_chunks(&p.g2);
+  p.narrow_kc1 = stream_chunk(p.g1.k, kAChunk / 64, kNarrowDepth);
+  p.half_kc4 = stream_chunk(p.g1.k, kAChunk / 256, 2);
+  return launch_kernel(small ? decode_pipeline_kernel<true> : decode_pipeline_kernel<false>,
+                       dim3(static_cast<unsigned>(num_cus)), dim3(kGemmThreads), kSmemBytes, stream, p);
 }
 
 hipError_t launch_grouped_gemm(const GemmArgs& g, int max_rows, int num_cus, hipStream_t stream,

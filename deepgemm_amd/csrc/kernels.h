@@ -90,6 +90,10 @@ struct GemmArgs {
   int num_experts;
   int n;
   int k;
+  // the STREAM engine's k-bytes a chunk and weight steps in flight for items of 1, 2 and 4 row tiles
+  // of 32 (set by the launch functions)
+  int kc[3];
+  int ring[3];
   GemmEngine engine;
   SwigluEpilogue sw;         // GEMM1 only (requires row_token); c is unused then
   int route_in_kernel;       // GEMM1: 1 = route the tasks in the kernel (<= gemm_route_max_tasks()),
@@ -193,18 +197,18 @@ hipError_t launch_combine(const CombineArgs& c, int num_cus, hipStream_t stream)
 
 // Decode pipeline (gemm.hip): GEMM1 with the in-kernel routing, the requant, GEMM2 of the
 // streaming engine and (PipeArgs::y) the combine in one launch, each group of rows handed from
-// GEMM1 to GEMM2 inside its XCD, each token combined once its experts' GEMM2 items are done.
+// GEMM1 to GEMM2, each token combined once its experts' GEMM2 items are done.
 // pipe: kPipeInts counters, zero when the launch starts (its last workgroup to leave zeroes
-// them again), each header counter in a 128-byte line of its own (every workgroup goes to them
-// at about the same time): the per-XCD claim counters at x * kPipeLine, the count of workgroups
-// that ran out of items at kPipeFinishAt, the count of workgroups that left at kPipeExitAt
+// them again), each XCD's header counters in a 128-byte line of their own (every workgroup goes to
+// them at about the same time): XCD x's claim counters at x * kPipeLine (GEMM1) and kPipeClaim2
+// ints further (GEMM2), the count of workgroups that left at kPipeExitAt
 // (the count of bounded waits that ran out next to it, at kPipeFailAt: rarely touched; the last
 // workgroup to leave copies it to meta[3]); then GEMM1 items done per group ([kPipeDone1At..],
 // kMaxPipeGroups) and GEMM2 items done per expert (expert e's at kPipeDone2At + e *
 // kPipeDone2Stride: the combine's waves poll them).
 constexpr int kPipeXcds = 8;
 constexpr int kPipeLine = 32;
-constexpr int kPipeFinishAt = kPipeXcds * kPipeLine;
+constexpr int kPipeClaim2 = kPipeLine / 2;
 constexpr int kPipeExitAt = (kPipeXcds + 1) * kPipeLine;
 constexpr int kPipeFailAt = kPipeExitAt + 1;
 // Polls of a bounded wait (a group's or an expert's count; far longer than any item). A wait
@@ -229,11 +233,14 @@ struct PipeArgs {
   int32_t* direct_flag;  // set to 0 (no direct rows), or null
   int32_t* pipe;
   uint16_t* y;           // non-null: the launch also runs the combine into y (bf16 [S, H];
-                         // H % 8 == 0 and H <= kPipeCombineMaxHidden)
+                         // H % 8 == 0)
   int spin_limit;        // polls of a bounded wait: kPipeSpinLimit, or 0 to test the error path
                          // (every wait then gives up at once)
+  // GEMM1's k-bytes a chunk in narrow items, and in items of 4 row tiles (half A chunk buffers, so
+  // that the accumulators leave registers for the loads); set by the launch function
+  int narrow_kc1;
+  int half_kc4;
 };
-constexpr int kPipeCombineMaxHidden = 64 * 8 * 8;  // one wave a token: 8 16-byte groups a lane
 bool decode_pipeline_supported(const GemmArgs& g1, const GemmArgs& g2, int num_cus);
 hipError_t launch_decode_pipeline(const PipeArgs& p, int num_cus, hipStream_t stream);
 

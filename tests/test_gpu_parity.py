@@ -720,6 +720,74 @@ def test_decode_pipeline_many_experts(mm, cuda, e, s, g):
     del l1, l2
 
 
+# (tokens, global experts or "zipf" or None for all local): the pipeline's small kernel (up to 320
+# tasks) with few, some and many experts touched (items of 2, 4 and 8 column units), at its largest
+# size, and with an expert of more rows than one of its 32-row chunks; the large kernel just above,
+# with 128-row groups in one round of items and with 64-row ones in two
+PIPE_CASES = {
+    "one_token": (1, None), "few": (8, 256), "some": (24, 256), "many": (53, None), "skewed": (48, "zipf"),
+    "large_kernel": (54, 256), "groups_128": (420, None), "groups_64": (341, "zipf"),
+}
+
+
+@pytest.mark.parametrize("case", list(PIPE_CASES))
+def test_decode_pipeline_item_shapes(mm, cuda, full_weights, case):
+    """Every stage against the oracle and the combine bitwise; then calls on the same buffer with
+    other inputs in turn, each bitwise a call on a fresh buffer (the rows that the items hand
+    over through memory are this call's, not an earlier one's)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the decode pipeline runs on the whole 256-CU MI355X only")
+    l1, l2, l1c, l2c, unpacked = full_weights
+    s, g = PIPE_CASES[case]
+    log(f"pipeline items {case}: S={s}")
+    kw = dict(routing="zipf") if g == "zipf" else dict(global_experts=g)
+    inputs = [make_tokens(s, 4096, 32, 6, seed=70 + s + i, **kw) for i in range(3)]
+    buf = mm.get_symm_buffer_for_mega_moe(None, 32, s, 6, 4096, 2048)
+    buf.scratch_view("pmax").fill_(-1.0)
+    y = run_layer(mm, buf, *inputs[0], l1, l2)
+    torch.cuda.synchronize()
+    tr = O.mega_moe_forward(*inputs[0], l1c, l2c, unpacked_weights=unpacked)
+    r = tr.routing.num_rows
+    assert bool((buf.scratch_view("pmax")[:r] >= 0).all()), "the pipeline ran"
+    if case == "skewed":
+        assert tr.routing.counts.max() > 32
+    if case == "groups_128":
+        assert tr.routing.counts.max() > 64
+    _stage_checks(buf, tr, s)
+    _combine_bitwise(mm, buf, y, l1, l2, s, None)
+    assert O.calc_diff(y.cpu(), tr.y) <= CALC_DIFF_BAR
+    fresh = []
+    for x in inputs:
+        fresh.append(run_layer(mm, mm.get_symm_buffer_for_mega_moe(None, 32, s, 6, 4096, 2048), *x, l1, l2).clone())
+    for i in range(12):
+        y = run_layer(mm, buf, *inputs[i % 3], l1, l2)
+        torch.cuda.synchronize()
+        assert mm.last_call_status(buf) == 0
+        assert torch.equal(y.view(torch.int16), fresh[i % 3].view(torch.int16)), f"call {i}"
+        assert torch.all(buf.scratch_view("pipe").cpu() == 0), "counters"
+
+
+@pytest.mark.parametrize("hdim,inter,s", [(7168, 2048, 16), (4096, 1536, 24), (2560, 512, 40), (640, 768, 30)])
+def test_decode_pipeline_small_other_shapes(mm, cuda, hdim, inter, s):
+    """The small kernel at other expert shapes (K in chunks that are not the LDS buffers' whole
+    length), and a hidden size it does not take (640: the separate launches)."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the decode pipeline runs on the whole 256-CU MI355X only")
+    e, k = 16, 8
+    log(f"small pipeline H={hdim} I={inter} S={s}")
+    x_fp8, x_sf, idx, w = make_tokens(s, hdim, e, k, seed=hdim + s, global_experts=64)
+    l1, l2 = make_weights_gpu(e, hdim, inter, seed=inter, mm=mm)
+    buf = mm.get_symm_buffer_for_mega_moe(None, e, s, k, hdim, inter)
+    buf.scratch_view("pmax").fill_(-1.0)
+    y = run_layer(mm, buf, x_fp8, x_sf, idx, w, l1, l2)
+    torch.cuda.synchronize()
+    tr = O.mega_moe_forward(x_fp8, x_sf, idx, w, *cpu_weights(l1, l2))
+    assert bool((buf.scratch_view("pmax")[:tr.routing.num_rows] >= 0).all()) == (hdim != 640)
+    _stage_checks(buf, tr, s)
+    _combine_bitwise(mm, buf, y, l1, l2, s, None)
+    assert O.calc_diff(y.cpu(), tr.y) <= CALC_DIFF_BAR
+
+
 def test_caller_scratch_reused_across_shapes(mm, cuda, full_weights):
     """One caller-owned route_scratch, zero-filled once, serves mmoe_forward calls of different
     shapes in turn through the C ABI: an all-local 1024-token call (6144 rows: its y spans
