@@ -365,6 +365,7 @@ int mmoe_forward_stages(const mmoe_forward_args* a, int first_stage, int last_st
   g1.row_token = at<int32_t>(ws, l.row_token_offset);
   g1.a_scale = a->x_sf;
   g1.lda = a->hidden;
+  g1.a_bytes = static_cast<int64_t>(a->num_tokens) * a->hidden;
   g1.b = static_cast<const uint8_t*>(a->w1);
   g1.b_scale = a->w1_sf;
   g1.c = nullptr;

@@ -5,12 +5,11 @@
 // (the dispatch "pull" of the reference's K1, megamoe/dcu_megamoe_large_opt/K1_fused/
 // k1_fused_ext.cu:479-746), so no grouped copy of x exists:
 //   h = bf16(acc * x_sf[token] * w1_sf[e, n])       for the gate and the up column of a channel
-// On the 8-wave kernel it fuses the K2 stage (megamoe/dcu_megamoe_large_opt/K2_fused/
+// It fuses the K2 stage (megamoe/dcu_megamoe_large_opt/K2_fused/
 // k2_fused_ext.cu:254-377) into its epilogue:
 //   y = silu(min(h_g, c)) * clamp(h_u, -c, c) * w    (fp32, left to right)
 // (each output tile holds matching gate and up channels, so SwiGLU is elementwise in
-// registers); on the WIDE kernel it writes h itself (bf16, the staged K1 output) and the
-// requant kernel computes y. The per-row requant (amax = max |y|; a = max(amax, 1e-4);
+// registers), on both kernels. The per-row requant (amax = max |y|; a = max(amax, 1e-4);
 // act = e4m3(clip(y * 448/a)); act_scale = a/448) needs the whole row and runs as its own small
 // kernel: a cross-workgroup hand-off inside GEMM1 would need an agent-scope release per tile,
 // which on gfx950 writes back the whole (per-XCD, non-coherent) L2 -- measured 4x slower than
@@ -29,7 +28,7 @@
 //      32) over the full K; wave w owns columns
 //      [64w, 64w + 64) and streams its weight columns from global memory into a register ring
 //      4 steps deep (Marlin gives each lane 16 contiguous k-bytes of one weight row; 16 lanes
-//      read 256 contiguous bytes), with no barrier: B never touches LDS. The A rows, the same
+//      read 256 contiguous bytes): B never touches LDS. The A rows, the same
 //      for the 8 waves, go to LDS once per workgroup in k-chunks of 64 KB loaded as whole
 //      128-byte lines, double buffered, one barrier per chunk (1-4 per tile). Loading A per
 //      wave in MFMA operand order (32 lines per instruction, re-read by every wave) made the A
@@ -37,13 +36,14 @@
 //    - TILE engine (more rows). A 256 x 256 output tile per workgroup, the 8 waves as 2 x 4
 //      with 128 x 64 each, K in 128-byte stages through double-buffered LDS (A rows
 //      XOR-swizzled, B in Marlin's own 256-byte blocks).
-//    Both engines let lane l supply k-bytes [32*(l/32), 32*(l/32)+32) of each 64-k MFMA step
+//    Both engines use the 32x32x64 MFMA, let lane l supply k-bytes [32*(l/32), 32*(l/32)+32) of each 64-k MFMA step
 //    for A and B alike and accumulate the 64-k steps in the same order.
 //  * the 4-wave WIDE kernel (every expert with many rows: prefill, MFMA-bound): one wave per
-//    SIMD with its 256 accumulators in AGPRs, 256 x 256 tiles, weights straight into
-//    registers and only A through LDS; described at wide_tile.
+//    SIMD with its 256 accumulators in AGPRs, 256 x 256 tiles of 16x16x128 MFMAs, weights straight
+//    into registers and only A through LDS; described at wide_tile.
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 #include "common.cuh"
 #include "kernels.h"
@@ -82,6 +82,23 @@ __device__ __forceinline__ v8i make_v8i(const int4& lo, const int4& hi) {
 
 __device__ __forceinline__ v16f mfma_fp8(const v8i& a, const v8i& b, const v16f& c) {
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+}
+
+// c += a b with the accumulator in AGPRs. Inline assembly: from the builtin the register allocator
+// moved some of a tile's 64 accumulators through VGPRs in the loop. The compiler does not see the
+// instruction's latency: read accumulators only after mfma_settle.
+__device__ __forceinline__ void mfma_fp8_16(const v8i& a, const v8i& b, v4f& c) {
+  asm("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+// The last MFMA's result (8 passes of 4 cycles) is in its registers before any of c is read.
+template <int N>
+__device__ __forceinline__ void mfma_settle(v4f (&c)[N][4]) {
+  asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < N; i += 2)
+    asm volatile("" : "+a"(c[i][0]), "+a"(c[i][1]), "+a"(c[i][2]), "+a"(c[i][3]), "+a"(c[i + 1][0]),
+                 "+a"(c[i + 1][1]), "+a"(c[i + 1][2]), "+a"(c[i + 1][3]));
 }
 
 __device__ __forceinline__ int4 ld16(const uint8_t* p) { return *reinterpret_cast<const int4*>(p); }
@@ -644,22 +661,30 @@ __device__ void tile_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, 
 // ------------------------------------------------------------------ WIDE engine
 // The TILE engine's 256 x 256 tile for a 4-wave workgroup (one wave per SIMD: 512 registers a
 // lane, the 256 accumulators in AGPRs), used when every expert has many rows. Wave w owns the
-// 64-column unit nb*4 + w over all 256 rows (8 x 2 MFMA tiles), so each weight column is read
+// 64-column unit nb*4 + w over all 256 rows (16 x 4 MFMA tiles), so each weight column is read
 // by one wave only: B goes straight from global memory into MFMA operand registers (Marlin
-// gives each lane 16 contiguous k-bytes of a weight row), four 64-k steps ahead in a register
-// ring, and never touches LDS. A goes through LDS in BK = 128 stages: 256 rows of 128 bytes,
+// gives each lane 16 contiguous k-bytes of a weight row), in a register ring of three 128-k stages,
+// and never touches LDS. A goes through LDS in BK = 128 stages: 256 rows of 128 bytes,
 // 16-byte piece p of row r at piece p ^ ((r / 2) % 8) (16 consecutive rows at one k hit 16
 // distinct 16-byte bank groups), three stages deep, so the first A operand of a stage is read
-// before the barrier that ends the previous one and the MFMA pipe does not drain there. A
-// stage's A is loaded one stage before its LDS write, spread one load or one LDS write per MFMA
-// group. Tiles are independent (prologue, stages, epilogue): a software pipeline across the
+// before the barrier that ends the previous one and the MFMA pipe does not drain there.
+// Tiles are independent (prologue, stages, epilogue): a software pipeline across the
 // tiles of a workgroup needed the next tile's offsets live through the stage loop and the
 // compiler spilled (measured slower).
+//
+// The MFMA is 16x16x128. At these sizes the chip is power-bound, and it takes less power for a FLOP
+// than 32x32x64: register-only loops over random e4m3 values sustain 4.43 against 4.05 PFLOP/s (over
+// zeros 4.97 and 4.96). Here the clock rises from 1.9 to 2.0 GHz, and a layer of 24.7K rows (4096 x
+// 4096, 4096 x 2048) goes from 703 to 689 us, of 49K Zipf rows from 1268 to 1256, of 196K rows from
+// 4845 to 4822; the results are the same bits. A first version with a two-stage ring (one burst of
+// loads a stage) was 1-3% slower than 32x32x64. Where the cycles are, by timing copies at 196K
+// rows: GEMM1 5.65 M, without A's and B's loads 4.5 M, without the LDS reads too 4.4 M (prologues and
+// epilogues then are 1.25 M of it), 3.15 M of MFMA.
 //
 // Two shapes (BM = rows of a full tile): BM = 256 with one workgroup per CU (512 registers a
 // lane), and BM = 128 with two workgroups per CU (256 registers a lane, 128 AGPR accumulators):
 // then each SIMD runs two waves of different tiles, and one tile's prologue and epilogue overlap
-// the other's MFMAs. The B ring and the A operand look-ahead are shallower at BM = 128 (the
+// the other's MFMAs. The A operand look-ahead is shallower at BM = 128 (the
 // other wave covers the latency).
 constexpr int kWideThreads = 256, kWideWaves = 4;
 constexpr int kWideBK = 128;
@@ -676,17 +701,16 @@ struct WideShape {
   static constexpr int kColScales = BM * 4;
   static constexpr int kAddrs = kColScales + kWideWaves * kStreamUnit * 4;
   static constexpr int kSmemBytes = kTables + kAddrs + BM * 8;
-  static constexpr int kRing = BM == 256 ? 4 : 2;  // 64-k steps of B in registers
   static constexpr int kWavesPerSimd = BM == 256 ? 1 : 2;
-  static constexpr int kFullTM = BM / 32;
+  static constexpr int kFullTM = BM / 16;
   // the epilogue stages each wave's 64 output rows (8 KB) in the A ring's first bytes
   static_assert(kWideWaves * 8192 <= kTables, "epilogue staging fits the A ring");
 };
 
 // Epilogue of a WIDE tile. The MFMAs run transposed (weights as the first operand), so lane
-// l holds token row tm*32 + l%32 and, per 32-column tile tn, the columns 8*(v/4) + 4*(l/32) +
-// v%4: four runs of 4 consecutive columns. The row scale is then one value per lane and row
-// tile, the column scales four 16-byte LDS reads per column tile (both from the tile's scale
+// l holds token row tm*16 + l%16 and, per 16-column tile tn, the 4 consecutive columns 4*(l/16) + v.
+// The row scale is then one value per lane and row
+// tile, the column scales one 16-byte LDS read per column tile (both from the tile's scale
 // table), and every 4 results become one 8-byte bf16 write into the wave's 8 KB slice of a
 // free 32 KB A buffer (64 rows x 128 bytes, 16-byte piece p of row r at p ^ ((r / 2) % 8):
 // conflict-free both ways); each pass of 64 rows then leaves as whole 16-byte pieces, 8 rows
@@ -694,46 +718,42 @@ struct WideShape {
 // GEMM2 writes the bf16 partials (-0 as +0) to the row addresses of the tile's table: its part
 // row, or for a row whose token has no other routed slot its y row (row_dest).
 template <int BM, int TM>
-__device__ __forceinline__ void store_wide(const GemmArgs& g, const v16f (&acc)[TM][2], int row0,
+__device__ __forceinline__ void store_wide(const GemmArgs& g, const v4f (&acc)[TM][4], int row0,
                                            int mrows, int unit, uint8_t* stage,
                                            const uint8_t* table) {
   using W = WideShape<BM>;
   const int tid = opaque_tid();
   const int lane = tid & (kWave - 1);
-  const int rl = lane & 31, hk = lane >> 5;
+  const int rl = lane & 15, q = lane >> 4;
   const float* s_xs = reinterpret_cast<const float*>(table);
   const float* s_bs = reinterpret_cast<const float*>(table + W::kColScales) + (tid / kWave) * kStreamUnit;
   const uint64_t* s_addr = reinterpret_cast<const uint64_t*>(table + W::kAddrs);
-  float4 bs[2][4];
+  float4 bs[4];
 #pragma unroll
-  for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) bs[tn][q] = *reinterpret_cast<const float4*>(s_bs + tn * 32 + q * 8 + hk * 4);
+  for (int tn = 0; tn < 4; ++tn) bs[tn] = *reinterpret_cast<const float4*>(s_bs + tn * 16 + q * 4);
   uint8_t* wlds = stage + (tid / kWave) * 8192;
   const int piece = lane & 7;
   const int col = unit * 64 + piece * 8;
 #pragma unroll
-  for (int pass = 0; pass < (TM + 1) / 2; ++pass) {
+  for (int pass = 0; pass < (TM + 3) / 4; ++pass) {
 #pragma unroll
-    for (int t2 = 0; t2 < (TM > 1 ? 2 : 1); ++t2) {  // TM = 1: one row tile, rows 32-63 unused
-      const int tm = pass * 2 + t2;
-      const float xs = s_xs[tm * 32 + rl];
-      const int r = t2 * 32 + rl;  // row within the pass
+    for (int t4 = 0; t4 < (TM < 4 ? TM : 4); ++t4) {  // (TM = 2: rows 32-63 unused)
+      const int tm = pass * 4 + t4;
+      const float xs = s_xs[tm * 16 + rl];
+      const int r = t4 * 16 + rl;  // row within the pass
       const int rkey = (r >> 1) & 7;
 #pragma unroll
-      for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float4 ws = bs[tn][q];
-          // the scale product as fma(., ., +0), the same rounding, but a zero is +0 (the
-          // combine's sum from +0 writes +0 too, so a y row written here matches it bitwise)
-          auto scaled = [&](float a, float w) { return __builtin_fmaf(a * xs, w, 0.0f); };
-          const uint32_t lo = pack_bf16x2(scaled(acc[tm][tn][4 * q], ws.x), scaled(acc[tm][tn][4 * q + 1], ws.y));
-          const uint32_t hi = pack_bf16x2(scaled(acc[tm][tn][4 * q + 2], ws.z), scaled(acc[tm][tn][4 * q + 3], ws.w));
-          // columns tn*32 + 8q + 4hk .. +4 -> bytes 64tn + 16q + 8hk: piece 4tn + q, half hk
-          const int pc = (4 * tn + q) ^ rkey;
-          *reinterpret_cast<uint2*>(wlds + r * 128 + pc * 16 + hk * 8) = make_uint2(lo, hi);
-        }
+      for (int tn = 0; tn < 4; ++tn) {
+        const float4 ws = bs[tn];
+        // the scale product as fma(., ., +0), the same rounding, but a zero is +0 (the
+        // combine's sum from +0 writes +0 too, so a y row written here matches it bitwise)
+        auto scaled = [&](float a, float w) { return __builtin_fmaf(a * xs, w, 0.0f); };
+        const uint32_t lo = pack_bf16x2(scaled(acc[tm][tn][0], ws.x), scaled(acc[tm][tn][1], ws.y));
+        const uint32_t hi = pack_bf16x2(scaled(acc[tm][tn][2], ws.z), scaled(acc[tm][tn][3], ws.w));
+        // columns 16tn + 4q .. +4 -> bytes 32tn + 8q: piece 2tn + q/2, half q%2
+        const int pc = (2 * tn + (q >> 1)) ^ rkey;
+        *reinterpret_cast<uint2*>(wlds + r * 128 + pc * 16 + (q & 1) * 8) = make_uint2(lo, hi);
+      }
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's LDS writes before its reads
     int4 val[8];
@@ -759,8 +779,8 @@ __device__ __forceinline__ void store_wide(const GemmArgs& g, const v16f (&acc)[
 }
 
 // Epilogue of a WIDE GEMM1 tile with the SwiGLU: the wave's unit holds the gate channels
-// unit*32 + c (column tile 0) and the up channels of the same c (column tile 1), so lane l has,
-// for token row tm*32 + l%32, four runs of 4 channels 8q + 4*(l/32) .. + 4 of both. Per channel:
+// unit*32 + c (column tiles 0, 1) and the up channels of the same c (column tiles 2, 3), so lane l
+// has, for token row tm*16 + l%16, two runs of 4 channels 16tn + 4*(l/16) .. + 4 of both. Per channel:
 // g = bf16(acc_g * x_scale * w_scale_g) and u = bf16(acc_u * x_scale * w_scale_u) (the staged
 // K1 output h, rounded like its stores), then y = SwiGLU(g, u) x route weight (the K2 formula,
 // with the activation clamp when kClamp) and y rounded to bf16: bf16 y [rows, I] for the
@@ -768,50 +788,48 @@ __device__ __forceinline__ void store_wide(const GemmArgs& g, const v16f (&acc)[
 // slice (64 rows x 64 bytes, 16-byte piece p of row r at p ^ ((r / 4) % 4)); a pass of 64 rows
 // leaves as 16-byte pieces, 16 rows per store instruction.
 template <bool kClamp, int BM, int TM>
-__device__ __forceinline__ void store_wide_swiglu(const GemmArgs& g, const v16f (&acc)[TM][2], int row0,
+__device__ __forceinline__ void store_wide_swiglu(const GemmArgs& g, const v4f (&acc)[TM][4], int row0,
                                                   int mrows, int unit, uint8_t* stage,
                                                   const uint8_t* table) {
   using W = WideShape<BM>;
   const int tid = opaque_tid();
   const int lane = tid & (kWave - 1);
-  const int rl = lane & 31, hk = lane >> 5;
+  const int rl = lane & 15, q = lane >> 4;
   const float* s_xs = reinterpret_cast<const float*>(table);
   const float* s_rw = reinterpret_cast<const float*>(table + W::kAddrs);  // route weights
   const float* s_bs = reinterpret_cast<const float*>(table + W::kColScales) + (tid / kWave) * kStreamUnit;
-  float4 bs[2][4];
+  float4 bs[4];
 #pragma unroll
-  for (int tn = 0; tn < 2; ++tn)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) bs[tn][q] = *reinterpret_cast<const float4*>(s_bs + tn * 32 + q * 8 + hk * 4);
+  for (int tn = 0; tn < 4; ++tn) bs[tn] = *reinterpret_cast<const float4*>(s_bs + tn * 16 + q * 4);
   uint8_t* wlds = stage + (tid / kWave) * 4096;
   const int64_t ld = g.sw.inter;
   uint16_t* out = g.sw.y + static_cast<int64_t>(row0) * ld + unit * 32 + (lane & 3) * 8;
   const float cv = g.sw.clamp;
 #pragma unroll
-  for (int pass = 0; pass < (TM + 1) / 2; ++pass) {
+  for (int pass = 0; pass < (TM + 3) / 4; ++pass) {
 #pragma unroll
-    for (int t2 = 0; t2 < (TM > 1 ? 2 : 1); ++t2) {  // TM = 1: one row tile, rows 32-63 unused
-      const int tm = pass * 2 + t2;
-      const float xs = s_xs[tm * 32 + rl];
-      const float rw = s_rw[tm * 32 + rl];
-      const int r = t2 * 32 + rl;  // row within the pass
+    for (int t4 = 0; t4 < (TM < 4 ? TM : 4); ++t4) {  // (TM = 2: rows 32-63 unused)
+      const int tm = pass * 4 + t4;
+      const float xs = s_xs[tm * 16 + rl];
+      const float rw = s_rw[tm * 16 + rl];
+      const int r = t4 * 16 + rl;  // row within the pass
       const int rkey = (r >> 2) & 3;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float4 wg = bs[0][q], wu = bs[1][q];
-        const v16f& ag = acc[tm][0];
-        const v16f& au = acc[tm][1];
+      for (int tn = 0; tn < 2; ++tn) {
+        const float4 wg = bs[tn], wu = bs[tn + 2];
+        const v4f& ag = acc[tm][tn];
+        const v4f& au = acc[tm][tn + 2];
         // gate and up of a channel rounded to bf16 together (one conversion for the pair)
         auto y_of = [&](float a_g, float a_u, float w_g, float w_u) {
           const uint32_t h = pack_bf16x2(a_g * xs * w_g, a_u * xs * w_u);
           return swiglu_weighted_c<kClamp>(__uint_as_float(h << 16), __uint_as_float(h & 0xffff0000u), rw, cv);
         };
-        const float y0 = y_of(ag[4 * q], au[4 * q], wg.x, wu.x);
-        const float y1 = y_of(ag[4 * q + 1], au[4 * q + 1], wg.y, wu.y);
-        const float y2 = y_of(ag[4 * q + 2], au[4 * q + 2], wg.z, wu.z);
-        const float y3 = y_of(ag[4 * q + 3], au[4 * q + 3], wg.w, wu.w);
-        // channels 8q + 4hk .. +4 -> bytes 16q + 8hk of the row: piece q, half hk
-        *reinterpret_cast<uint2*>(wlds + r * 64 + ((q ^ rkey) << 4) + hk * 8) =
+        const float y0 = y_of(ag[0], au[0], wg.x, wu.x);
+        const float y1 = y_of(ag[1], au[1], wg.y, wu.y);
+        const float y2 = y_of(ag[2], au[2], wg.z, wu.z);
+        const float y3 = y_of(ag[3], au[3], wg.w, wu.w);
+        // channels 16tn + 4q .. +4 -> bytes 32tn + 8q of the row: piece 2tn + q/2, half q%2
+        *reinterpret_cast<uint2*>(wlds + r * 64 + (((2 * tn + (q >> 1)) ^ rkey) << 4) + (q & 1) * 8) =
             make_uint2(pack_bf16x2(y0, y1), pack_bf16x2(y2, y3));
       }
     }
@@ -831,29 +849,37 @@ __device__ __forceinline__ void store_wide_swiglu(const GemmArgs& g, const v16f 
   }
 }
 
-// TM row tiles of 32: BM/32 for a full tile; fewer (4, 2 or 1) for an expert's last tile of
+// TM row tiles of 16: BM/16 for a full tile; fewer (8, 4 or 2) for an expert's last tile of
 // at most 128, 64 or 32 rows (a fraction of the MFMAs and A traffic for the row remainder).
-template <bool kGather, bool kSwiglu, int BM, int TM, typename Hook = NoHook>
+//
+// The stage loop is unrolled by 3, so that the LDS buffer, the B ring slot and the A registers of a
+// stage are fixed. At stage kt every even group writes one piece of stage kt + 2's A to LDS and loads,
+// into the same registers, the piece 1.5 stages further on; the odd groups of the first half
+// load stage kt + 2's weights into the ring slot that stage kt - 1 has left. Spread out like that, the
+// loads and LDS writes issue in the gaps between MFMAs instead of stalling the MFMA pipe in
+// bursts, and every load has at least a stage and a half (~1.5 us) to arrive.
+//
+// kBig: the token matrix spans 4 GB or more (GEMM1's gathered rows need 64-bit offsets).
+template <bool kGather, bool kSwiglu, int BM, int TM, bool kBig, typename Hook = NoHook>
 __device__ void wide_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, int mrows, int nb,
                           uint8_t* smem, const Hook& before_epilogue = Hook{}) {
   using W = WideShape<BM>;
+  using Offset = std::conditional_t<kBig, uint64_t, uint32_t>;
   constexpr int kWideStage = W::kStage;
   constexpr int kWideTables = W::kTables;
-  constexpr int kWideRing = W::kRing;
-  static_assert(TM <= W::kFullTM, "a tile of at most BM rows");
-  constexpr int TN = kStreamUnit / 32;                        // 2
-  constexpr int kALoads = TM * 32 * kWideBK / 16 / kWideThreads;  // TM
+  static_assert(TM <= W::kFullTM && TM >= 2, "a tile of at most BM rows");
+  constexpr int TN = kStreamUnit / 16;                            // 4
+  constexpr int kALoads = TM * 16 * kWideBK / 16 / kWideThreads;  // TM / 2
   constexpr int kRowsPerLoad = kWideThreads / (kWideBK / 16);     // 32
   const int tid = opaque_tid();
   const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int stages = g.k / kWideBK;
-  const int steps = stages * (kWideBK / 64);
   const int units = g.n / kStreamUnit;
   const int unit_raw = nb * kWideWaves + wave;
   const bool active = unit_raw < units;
   const int unit = active ? unit_raw : units - 1;  // a partial column block: any valid columns
-  const int hk = lane >> 5;
+  const int q = lane >> 4;
 
   // A: load i covers row i*32 + tid/8, piece tid % 8 (rows past mrows read row 0). GEMM1
   // (gather): the row scales for the epilogue's table are loaded by the same threads, from the
@@ -862,111 +888,103 @@ __device__ void wide_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, 
   // the stages' loads, so that every wait the compiler places in the prologue is exact (a scale
   // chain of its own, token -> scale, had been sunk behind all the stage loads and made the
   // prologue wait for every one of them). GEMM2 loads one row scale a thread (no chain).
-  const uint8_t* a_src[kALoads];
+  const uint8_t* const a_base = kGather ? g.a : g.a + static_cast<int64_t>(row0) * g.lda;
+  Offset a_off[kALoads];
   float a_rs[kALoads];
-  int64_t a_row[kALoads];
+  int a_row[kALoads];
 #pragma unroll
   for (int i = 0; i < kALoads; ++i) {
     const int r = i * kRowsPerLoad + (tid >> 3);
-    const int row = row0 + (r < mrows ? r : 0);
-    a_row[i] = kGather ? static_cast<int64_t>(rs.token(row)) : row;
+    const int row = r < mrows ? r : 0;
+    a_row[i] = kGather ? rs.token(row0 + row) : row;
   }
 #pragma unroll
   for (int i = 0; i < kALoads; ++i) {
-    a_src[i] = g.a + a_row[i] * g.lda + (tid & 7) * 16;
+    a_off[i] = static_cast<Offset>(a_row[i]) * static_cast<Offset>(g.lda) + (tid & 7) * 16;
     a_rs[i] = kGather ? g.a_scale[a_row[i]] : 0.0f;
   }
   const float pre_xs = kGather ? 0.0f : g.a_scale[row0 + min(tid, mrows - 1)];
   const int a_dst0 = (tid >> 3) * kWideBK + (((tid & 7) ^ ((tid >> 4) & 7)) << 4);
-  // two register sets: a stage's A is loaded one stage before it is written to LDS, which is
-  // one stage before it is read
-  int4 ra[2][kALoads];
-  auto load_a = [&](int set, int i, int kt) { ra[set][i] = ld16(a_src[i] + kt * kWideBK); };
-  auto store_a = [&](int set, int i, int kt) {
-    *reinterpret_cast<int4*>(smem + (kt % kWideBufs) * kWideStage + a_dst0 + i * kRowsPerLoad * kWideBK) =
-        ra[set][i];
+  auto fetch_a = [&](int i, int kt) { return ld16(a_base + kt * kWideBK + a_off[i]); };
+  // piece i of stage kt in buffer `buf` (kt % 3)
+  auto put_a = [&](int buf, int i, const int4& v) {
+    *reinterpret_cast<int4*>(smem + buf * kWideStage + a_dst0 + i * kRowsPerLoad * kWideBK) = v;
   };
-  // B: column tile tn of the wave's unit; 64-k step s of the lane's column at + s*1024 (+256)
+  // Pieces in flight: piece i of stage kt in slot (kt * kALoads + i) % kSlots, the same for kt and
+  // kt + 3. kDelay pieces lie between a slot's LDS write and its next load: 1.5 stages (TM = 2: 2).
+  constexpr int kDelay = TM == 2 ? 2 : kALoads + kALoads / 2;
+  constexpr int kSlots = TM == 2 ? 3 : kDelay;
+  static_assert(3 * kALoads % kSlots == 0, "slots repeat with the unrolled stages");
+  int4 ra[kSlots];
+  // B: column tile tn (16 columns) of the wave's unit, stage s at + s * 2048: lane l has column l % 16
+  // and the 16-byte k-blocks l/16 and l/16 + 4 of the stage's eight (A's operands the same, so the
+  // order of k inside the MFMA is the caller's to choose: a load is 1 KB contiguous)
   const uint8_t* bp[TN];
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn) {
-    const int n = weight_row<kSwiglu>(g, unit, kStreamUnit, tn * 32 + (lane & 31));
-    bp[tn] = g.b + (static_cast<int64_t>(e) * (g.n / 16) + (n >> 4)) * (static_cast<int64_t>(g.k) * 16) +
-             (n & 15) * 16 + hk * 512;
+    const int n = weight_row<kSwiglu>(g, unit, kStreamUnit, tn * 16);
+    bp[tn] = g.b + (static_cast<int64_t>(e) * (g.n / 16) + (n >> 4)) * (static_cast<int64_t>(g.k) * 16);
   }
-  int4 br[kWideRing][TN][2];
-  auto load_b = [&](int slot, int s) {
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const uint8_t* q = bp[tn] + static_cast<int64_t>(s) * 1024;
-      br[slot][tn][0] = ld16(q);
-      br[slot][tn][1] = ld16(q + 256);
-    }
+  int4 br[3][TN][2];
+  const uint32_t b_off = lane * 16;
+  auto load_b = [&](int slot, int j, int s) {  // half j % 2 of tile j / 2
+    br[slot][j / 2][j % 2] = ld16(bp[j / 2] + static_cast<int64_t>(s) * 2048 + (j % 2) * 1024 + b_off);
   };
 
-  v16f acc[TM][TN];
+  v4f acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+      for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.0f;
 
-  const int rkey = ((lane & 31) >> 1) & 7;
-  auto read_a = [&](int kt, int ks, int tm) {
-    const int p0 = ks * 4 + hk * 2;
-    const uint8_t* ar = smem + (kt % kWideBufs) * kWideStage + (tm * 32 + (lane & 31)) * kWideBK;
-    return make_v8i(*reinterpret_cast<const int4*>(ar + ((p0 ^ rkey) << 4)),
-                    *reinterpret_cast<const int4*>(ar + (((p0 + 1) ^ rkey) << 4)));
+  const int rkey = ((lane & 15) >> 1) & 7;
+  const uint8_t* const a_read = smem + (lane & 15) * kWideBK + ((q ^ rkey) << 4);
+  const uint8_t* const a_read4 = smem + (lane & 15) * kWideBK + (((q ^ rkey) << 4) ^ 64);
+  auto read_a = [&](int buf, int tm) {
+    const int at = buf * kWideStage + tm * 16 * kWideBK;
+    return make_v8i(*reinterpret_cast<const int4*>(a_read + at), *reinterpret_cast<const int4*>(a_read4 + at));
   };
-  // A stage = 16 MFMA groups (2 steps x 8 row tiles, 2 MFMAs each). The A operand of group
+  // A stage = 16 MFMA groups (16 row tiles, 4 MFMAs each). The A operand of group
   // g + 3 is read while group g's MFMAs run (ring of 4 operands; the last groups read the next
   // stage's first operands, whose buffer is complete since the previous barrier), which
   // covers the LDS latency with one wave per SIMD. Order pinned by sched_barrier.
-  constexpr int kGroups = (kWideBK / 64) * TM;
-  // one wave a SIMD: read 3 groups ahead; two (BM = 128): 1; TM = 1 has two groups a stage
+  constexpr int kGroups = TM;
+  // one wave a SIMD: read 3 groups ahead; two (BM = 128): 1; TM = 2 has two groups a stage
   constexpr int kAhead = W::kWavesPerSimd == 1 ? (kGroups >= 4 ? 3 : kGroups - 1) : 1;
   static_assert(kGroups % (kAhead + 1) == 0, "operand ring index must repeat per stage");
   v8i abuf[kAhead + 1];
-  auto read_group = [&](int kt, int gi) {
-    const int g2 = gi % kGroups;
-    return read_a(kt + gi / kGroups, g2 / TM, g2 % TM);
-  };
-  const int last_step = steps - 1;
   const int last_stage = stages - 1;
-  // stage kt: 16 groups; groups 0-7 each load one piece of stage kt + 3's A into register set
-  // `lset`, groups 8-15 each write one piece of stage kt + 2's A (set `wset`, loaded during
-  // the previous stage) into its LDS buffer, each step's last group refills its B ring slot
-  // with the step 4 ahead; then the barrier. Spread out, these loads and LDS writes issue in
-  // the gaps between MFMAs instead of stalling the MFMA pipe in bursts.
-  auto stage = [&](int kt, int slot0, int wset, int lset) {
-    const int kt_load = min(kt + 3, last_stage);
+  constexpr int kBGroups = (TM < 8 ? TM : 8) / 2;  // odd groups that load weights
+  // stage kt; ph = kt % 3 (a constant)
+  auto stage = [&](int kt, int ph) {
 #pragma unroll
     for (int gi = 0; gi < kGroups; ++gi) {
-      const int ks = gi / TM, tm = gi % TM;
-      abuf[(gi + kAhead) % (kAhead + 1)] = read_group(kt, gi + kAhead);
-      if (gi < kALoads) load_a(lset, gi, kt_load);
-      else store_a(wset, gi - kALoads, kt + 2);
+      const int ahead = gi + kAhead;
+      abuf[ahead % (kAhead + 1)] = read_a((ph + ahead / kGroups) % 3, ahead % kGroups);
+      if (gi % 2 == 0) {
+        const int i = gi / 2, n = (ph + 2) * kALoads + i;
+        put_a((ph + 2) % 3, i, ra[n % kSlots]);
+        ra[(n + kDelay) % kSlots] = fetch_a((i + kDelay) % kALoads, min(kt + 2 + (i + kDelay) / kALoads, last_stage));
+      } else if (gi / 2 < kBGroups) {
+#pragma unroll
+        for (int j = gi / 2 * (2 * TN / kBGroups); j < (gi / 2 + 1) * (2 * TN / kBGroups); ++j)
+          load_b((ph + 2) % 3, j, min(kt + 2, last_stage));
+      }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn)
-        acc[tm][tn] = mfma_fp8(make_v8i(br[slot0 + ks][tn][0], br[slot0 + ks][tn][1]),
-                               abuf[gi % (kAhead + 1)], acc[tm][tn]);  // transposed tile
+        mfma_fp8_16(make_v8i(br[ph][tn][0], br[ph][tn][1]), abuf[gi % (kAhead + 1)], acc[gi][tn]);  // transposed tile
       __builtin_amdgcn_sched_barrier(0);
-      if (tm == TM - 1) {
-        load_b(slot0 + ks, min(kt * (kWideBK / 64) + ks + kWideRing, last_step));
-        __builtin_amdgcn_sched_barrier(0);
-      }
     }
     lds_barrier();
   };
-  static_assert(kGroups == 2 * kALoads, "one A load and one A write per group");
 
   // prologue: the epilogue's scales (the row scales loaded with the row tokens above; thread
-  // t: the weight-row scale of its wave's column lane), A stages 0 and 1 into LDS, stage 2 into
-  // register set 0, B steps 0..3, the first operands; the loads of stages 0, 1 and 2 go out
-  // together (stage 0 through registers of the prologue's own), so that stage 2 is in before
-  // the first stage needs it.
+  // t: the weight-row scale of its wave's column lane), A stages 0 and 1 into LDS, the pieces of the
+  // next 1.5 stages into their registers, B stages 0 and 1, the first operands; the loads
+  // go out together (stages 0 and 1 through registers of the prologue's own).
   // GEMM2: row tid's output address (its part row, or its token's y row when the token has no
   // other routed slot and direct rows are on); the switch and the row table load side by side.
   // Rows past mrows take the last row's (never stored).
@@ -978,20 +996,22 @@ __device__ void wide_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, 
   // GEMM1: row tid's route weight (the SwiGLU epilogue's)
   const float pre_rw = kSwiglu ? g.sw.row_weight[row0 + min(tid, mrows - 1)] : 0.0f;
   const float pre_bs = g.b_scale[static_cast<int64_t>(e) * g.n + weight_row<kSwiglu>(g, unit, kStreamUnit, lane)];
-  int4 ra0[kALoads];
+  int4 ra0[2][kALoads];
 #pragma unroll
-  for (int i = 0; i < kALoads; ++i) ra0[i] = ld16(a_src[i]);
+  for (int i = 0; i < kALoads; ++i) ra0[0][i] = fetch_a(i, 0);
 #pragma unroll
-  for (int i = 0; i < kALoads; ++i) load_a(1, i, min(1, last_stage));
+  for (int i = 0; i < kALoads; ++i) ra0[1][i] = fetch_a(i, min(1, last_stage));
 #pragma unroll
-  for (int i = 0; i < kALoads; ++i) load_a(0, i, min(2, last_stage));
+  for (int j = 0; j < 2 * TN; ++j) load_b(0, j, 0);
 #pragma unroll
-  for (int sl = 0; sl < kWideRing; ++sl) load_b(sl, min(sl, last_step));
+  for (int n = 2 * kALoads; n < 2 * kALoads + kDelay; ++n)
+    ra[n % kSlots] = fetch_a(n % kALoads, min(n / kALoads, last_stage));
 #pragma unroll
-  for (int i = 0; i < kALoads; ++i)
-    *reinterpret_cast<int4*>(smem + a_dst0 + i * kRowsPerLoad * kWideBK) = ra0[i];  // stage 0, buffer 0
+  for (int j = 0; j < 2 * TN; ++j) load_b(1, j, min(1, last_stage));
 #pragma unroll
-  for (int i = 0; i < kALoads; ++i) store_a(1, i, 1);
+  for (int i = 0; i < kALoads; ++i) put_a(0, i, ra0[0][i]);
+#pragma unroll
+  for (int i = 0; i < kALoads; ++i) put_a(1, i, ra0[1][i]);
   if constexpr (kGather) {
 #pragma unroll
     for (int i = 0; i < kALoads; ++i) reinterpret_cast<float*>(smem + kWideTables)[i * kRowsPerLoad + (tid >> 3)] = a_rs[i];
@@ -1008,16 +1028,20 @@ __device__ void wide_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, 
   }
   lds_barrier();
 #pragma unroll
-  for (int gi = 0; gi < kAhead; ++gi) abuf[gi] = read_group(0, gi);
-  // two stages per iteration, so that the ring slots are compile-time indices; every load is
-  // issued unconditionally (past the end it reloads the last step or stage), which keeps the
+  for (int gi = 0; gi < kAhead; ++gi) abuf[gi] = read_a(gi / kGroups, gi % kGroups);
+  // every load is issued unconditionally (past the end it reloads the last stage), which keeps the
   // compiler's load counting exact
-  for (int kt = 0; kt < stages; kt += 2) {  // stages is even (k % 256 == 0)
-    stage(kt, 0, 0, 1);
-    stage(kt + 1, kWideRing == 4 ? 2 : 0, 1, 0);  // a ring of 2 refills the same two slots
+  int kt = 0;
+  for (; kt + 3 <= stages; kt += 3) {
+    stage(kt, 0);
+    stage(kt + 1, 1);
+    stage(kt + 2, 2);
   }
+  if (kt < stages) stage(kt, 0);
+  if (kt + 1 < stages) stage(kt + 1, 1);
   // every wave has passed its last LDS read of A (the barrier that ended the last stage)
   before_epilogue();
+  mfma_settle(acc);
   if (!active) return;
   if constexpr (kSwiglu) {
     if (g.sw.has_clamp) store_wide_swiglu<true, BM, TM>(g, acc, row0, mrows, unit, smem, smem + kWideTables);
@@ -1894,7 +1918,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
 
 // Persistent dispatcher of the WIDE engine: every expert's rows as BM x 256 tiles, items dealt
 // to the XCDs in contiguous ranges like the 8-wave dispatcher's.
-template <bool kGather, bool kSwiglu, int BM>
+template <bool kGather, bool kSwiglu, int BM, bool kBig>
 __global__ __launch_bounds__(kWideThreads, WideShape<BM>::kWavesPerSimd) void wide_gemm_kernel(GemmArgs g) {
   if (dual_skips(g, true)) return;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -1915,19 +1939,19 @@ __global__ __launch_bounds__(kWideThreads, WideShape<BM>::kWavesPerSimd) void wi
   const RowSrc rs{g.row_token, g.sw.row_weight, 0};
   auto run_item = [&](int t, const auto& before_epilogue) {
     const int e = expert_of_item(s_prefix, E, t);
-    const int cnt = s_count[e];
+    const int cnt = __builtin_amdgcn_readfirstlane(s_count[e]);
     int mt, nb;
-    tile_coords(t - s_prefix[e], cnt, tile_nb, mt, nb, BM);
+    tile_coords(t - __builtin_amdgcn_readfirstlane(s_prefix[e]), cnt, tile_nb, mt, nb, BM);
     const int mrows = min(BM, cnt - mt * BM);
-    const int row0 = s_off[e] + mt * BM;
+    const int row0 = __builtin_amdgcn_readfirstlane(s_off[e]) + mt * BM;
     if (BM == 256 && mrows > 128)
-      wide_tile<kGather, kSwiglu, BM, (BM == 256 ? 8 : 4)>(g, rs, e, row0, mrows, nb, smem, before_epilogue);
+      wide_tile<kGather, kSwiglu, BM, BM / 16, kBig>(g, rs, e, row0, mrows, nb, smem, before_epilogue);
     else if (mrows > 64)
-      wide_tile<kGather, kSwiglu, BM, 4>(g, rs, e, row0, mrows, nb, smem, before_epilogue);
+      wide_tile<kGather, kSwiglu, BM, 8, kBig>(g, rs, e, row0, mrows, nb, smem, before_epilogue);
     else if (mrows > 32)
-      wide_tile<kGather, kSwiglu, BM, 2>(g, rs, e, row0, mrows, nb, smem, before_epilogue);
+      wide_tile<kGather, kSwiglu, BM, 4, kBig>(g, rs, e, row0, mrows, nb, smem, before_epilogue);
     else
-      wide_tile<kGather, kSwiglu, BM, 1>(g, rs, e, row0, mrows, nb, smem, before_epilogue);
+      wide_tile<kGather, kSwiglu, BM, 2, kBig>(g, rs, e, row0, mrows, nb, smem, before_epilogue);
   };
   // One item at a time from the static deal or from the claims. Claiming only pays when a
   // workgroup has few items (the last round's granularity is then a large share of its work;
@@ -1951,7 +1975,7 @@ __global__ __launch_bounds__(kWideThreads, WideShape<BM>::kWavesPerSimd) void wi
   while (true) {
     int t;
     if (dynamic) {
-      t = s_item;
+      t = __builtin_amdgcn_readfirstlane(s_item);
     } else {
       for (t = -1; k < deal.rounds() && t < 0; ++k) {
         const int c = deal.item(k);
@@ -2034,18 +2058,18 @@ hipError_t ensure_dynamic_lds(int bytes) {
   return err;
 }
 
-template <bool kGather, bool kSwiglu, int BM>
+template <bool kGather, bool kSwiglu, int BM, bool kBig = false>
 hipError_t launch_wide(const GemmArgs& g, int max_rows, int num_cus, hipStream_t stream) {
   using W = WideShape<BM>;
   {  // the dynamic LDS (up to 104 KB) exceeds the default limit
-    const hipError_t err = ensure_dynamic_lds<&wide_gemm_kernel<kGather, kSwiglu, BM>>(W::kSmemBytes);
+    const hipError_t err = ensure_dynamic_lds<&wide_gemm_kernel<kGather, kSwiglu, BM, kBig>>(W::kSmemBytes);
     if (err != hipSuccess) return err;
   }
   const int64_t bound =
       (static_cast<int64_t>(max_rows) / BM + g.num_experts) * ((g.n + kTileBN - 1) / kTileBN);
   int64_t grid = static_cast<int64_t>(num_cus) * W::kWavesPerSimd;  // workgroups a CU: 1 or 2
   if (grid > bound) grid = bound;
-  return launch_kernel(wide_gemm_kernel<kGather, kSwiglu, BM>, dim3(static_cast<unsigned>(grid)),
+  return launch_kernel(wide_gemm_kernel<kGather, kSwiglu, BM, kBig>, dim3(static_cast<unsigned>(grid)),
                        dim3(kWideThreads), W::kSmemBytes, stream, g);
 }
 
@@ -2195,6 +2219,13 @@ hipError_t launch_decode_pipeline(const PipeArgs& args, int num_cus, hipStream_t
                        dim3(static_cast<unsigned>(num_cus)), dim3(kGemmThreads), kSmemBytes, stream, p);
 }
 
+static hipError_t launch_wide_gemm(const GemmArgs& g, int max_rows, int num_cus, hipStream_t stream) {
+  if (!g.sw.enabled) return launch_wide<false, false, kWideBM2>(g, max_rows, num_cus, stream);
+  // 32-bit offsets into the token matrix (8 registers and an addition a load less) up to 4 GB
+  return g.a_bytes >= int64_t{1} << 32 ? launch_wide<true, true, kWideBM1, true>(g, max_rows, num_cus, stream)
+                                       : launch_wide<true, true, kWideBM1>(g, max_rows, num_cus, stream);
+}
+
 hipError_t launch_grouped_gemm(const GemmArgs& g, int max_rows, int num_cus, hipStream_t stream,
                                const int32_t* rows_on_device, bool route_small_in_kernel,
                                int dual_min_rows) {
@@ -2231,15 +2262,12 @@ hipError_t launch_grouped_gemm(const GemmArgs& g, int max_rows, int num_cus, hip
     const hipError_t err = g.sw.enabled ? launch_engines<true, true>(eight, max_rows, num_cus, stream)
                                         : launch_engines<false, false>(eight, max_rows, num_cus, stream);
     if (err != hipSuccess) return err;
-    return g.sw.enabled ? launch_wide<true, true, kWideBM1>(d, max_rows, num_cus, stream)
-                        : launch_wide<false, false, kWideBM2>(d, max_rows, num_cus, stream);
+    return launch_wide_gemm(d, max_rows, num_cus, stream);
   }
   if (wide && route_small_in_kernel) return hipErrorInvalidValue;  // (rows_on_device is set)
-  if (g.sw.enabled)
-    return wide ? launch_wide<true, true, kWideBM1>(g, max_rows, num_cus, stream)
-                : launch_engines<true, true>(eight, max_rows, num_cus, stream);
-  return wide ? launch_wide<false, false, kWideBM2>(g, max_rows, num_cus, stream)
-              : launch_engines<false, false>(eight, max_rows, num_cus, stream);
+  if (wide) return launch_wide_gemm(g, max_rows, num_cus, stream);
+  return g.sw.enabled ? launch_engines<true, true>(eight, max_rows, num_cus, stream)
+                      : launch_engines<false, false>(eight, max_rows, num_cus, stream);
 }
 
 }  // namespace mmoe

@@ -82,6 +82,7 @@ struct GemmArgs {
   const int32_t* row_token;  // non-null: A row r is a[row_token[r]] (gather), scale a_scale[token]
   const float* a_scale;      // per token (gather) or per row
   int64_t lda;
+  int64_t a_bytes;           // GEMM1: the token matrix's size
   const uint8_t* b;          // e4m3 Marlin [E, N/16, K*16]
   const float* b_scale;      // f32 [E, N]
   uint16_t* c;               // bf16 [rows, N]

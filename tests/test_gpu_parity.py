@@ -632,6 +632,60 @@ def test_layer_prefill_full_scale_sampled(mm, cuda, full_weights, cfg):
     assert torch.equal(y1, y), "two calls bitwise identical"
 
 
+@pytest.mark.parametrize("hdim,inter", [(512, 256), (768, 512), (1024, 768)])
+def test_wide_tile_heights(mm, cuda, hdim, inter):
+    """Last row blocks on both sides of every WIDE tile height (1, 32 | 33, 64 | 65, 128 | 129, 256
+    rows) at K of 2 to 8 stages (every remainder of the stage loop unrolled by 3): each expert has
+    1024 rows and such a block."""
+    e, tails = 8, (1, 32, 33, 64, 65, 128, 129, 256)
+    idx = torch.cat([torch.full((1024 + t,), i, dtype=torch.int64) for i, t in enumerate(tails)])
+    gen = torch.Generator().manual_seed(hdim)
+    idx = idx[torch.randperm(idx.numel(), generator=gen)].view(-1, 1).contiguous()
+    s = idx.shape[0]
+    w = torch.rand((s, 1), generator=gen) + 0.05
+    x_fp8, x_sf = O.cast_to_fp8_channelwise(torch.randn((s, hdim), generator=gen).to(torch.bfloat16))
+    l1, l2 = make_weights_gpu(e, hdim, inter, seed=inter, mm=mm)
+    buf = mm.SymmBuffer(None, e, s, 1, hdim, inter)
+    log(f"WIDE tile heights H={hdim} I={inter} S={s}")
+    y = run_layer(mm, buf, x_fp8, x_sf, idx, w, l1, l2, clamp=2.0)
+    torch.cuda.synchronize()
+    assert buf.scratch_view("meta")[1].item() == 1 and buf.scratch_view("meta")[2].item() == 1
+    tr = O.mega_moe_forward(x_fp8, x_sf, idx, w, *cpu_weights(l1, l2), activation_clamp=2.0)
+    _stage_checks(buf, tr, s, 2.0)
+    _combine_bitwise(mm, buf, y, l1, l2, s, 2.0)
+    assert O.calc_diff(y.cpu(), tr.y) <= CALC_DIFF_BAR
+
+
+def test_wide_token_matrix_over_4gb(mm, cuda):
+    """A token matrix of more than 4 GB: the WIDE GEMM1 gathers its rows with 64-bit offsets.
+    Sampled tokens at both ends and on both sides of the 4 GB line against the oracle."""
+    s, e, hdim, inter = 1_048_600, 4, 4096, 256
+    log("WIDE beyond 4 GB of tokens")
+    buf = mm.SymmBuffer(None, e, s, 1, hdim, inter)
+    g = torch.Generator(device="cuda").manual_seed(3)
+    for b in range(0, s, 1 << 16):
+        n = min(1 << 16, s - b)
+        q, sf = mm.cast_to_fp8_channelwise(torch.randn((n, hdim), generator=g, device="cuda").to(torch.bfloat16))
+        buf.x[b:b + n].copy_(q)
+        buf.x_sf[b:b + n].copy_(sf)
+    buf.topk_idx.copy_(torch.randint(0, e, (s, 1), generator=g, device="cuda"))
+    buf.topk_weights.copy_(torch.rand((s, 1), generator=g, device="cuda") + 0.05)
+    l1, l2 = make_weights_gpu(e, hdim, inter, seed=9, mm=mm)
+    y = torch.empty((s, hdim), dtype=torch.bfloat16, device=cuda)
+    mm.fp8_w8a8_mega_moe(y, l1, l2, buf)
+    torch.cuda.synchronize()
+    assert buf.scratch_view("meta")[1].item() == 1
+    line = (1 << 32) // hdim
+    sel = torch.tensor([0, 1, 77, line - 2, line - 1, line, line + 1, s - 2, s - 1], device=cuda)
+    xs = buf.x.view(torch.uint8)[sel].cpu().view(torch.float8_e4m3fn)
+    tr = O.mega_moe_forward(xs, buf.x_sf[sel].cpu(), buf.topk_idx[sel].cpu(), buf.topk_weights[sel].cpu(),
+                            *cpu_weights(l1, l2))
+    for i in range(sel.numel()):
+        assert O.calc_diff(y[sel[i]].cpu(), tr.y[i]) <= CALC_DIFF_BAR, int(sel[i])
+    del buf, y
+    torch.cuda.empty_cache()
+
+
 def test_wide_claim_counters_return_to_zero(mm, cuda):
     """The WIDE GEMMs claim items from per-XCD counters in route_scratch when a workgroup has few
     items; the last workgroup of each GEMM resets them, so after a call (and after a GEMM2 run on
