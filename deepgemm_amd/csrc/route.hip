@@ -13,9 +13,9 @@
 // popcount of that mask below it and the group's lowest lane publishes the group size. Per-wave
 // counts become per-wave bases through LDS prefix sums.
 //
-// Two launch shapes, both integer work bound by the topk tables' HBM reads:
-//   * small (<= 16384 tasks): ONE workgroup of 16 waves does count, scan and scatter;
-//   * large: a count kernel (one workgroup per chunk, LDS histogram) and a scatter kernel
+// Two launch shapes, both integer work bound by the topk tables' reads and their latency:
+//   * up to 24576 tasks: one launch with a workgroup for each expert, which ranks that expert's tasks;
+//   * more: a count kernel (one workgroup per chunk, LDS histogram) and a scatter kernel
 //     (one workgroup per chunk) that rebuilds the expert offsets and its chunk base from the
 //     per-chunk counts itself, so no grid-wide barrier or separate scan launch is needed.
 #include "launch.h"
@@ -25,9 +25,16 @@ namespace mmoe {
 
 namespace {
 
-constexpr int kSmallThreads = 1024;
-constexpr int kSmallWaves = kSmallThreads / kWave;
-constexpr int kSmallMaxExperts = 256;
+constexpr int kExpertThreads = 1024;
+constexpr int kExpertWaves = kExpertThreads / kWave;
+constexpr int kExpertMaxExperts = 256;
+// Tasks up to which a workgroup an expert routes: it reads all of them, so its time grows with their
+// number, while the chunk kernels' two launches have a floor of 17 us. 32 experts, us (one of 8 slots
+// local / all of them local): 8192 tasks 5.6 / 7.2, 16384 8.3 / 11.6, 24576 10.4 / 16.1, 32768
+// 12.6 / 19.9, against the chunk kernels' 17 / 17 (24576) and 17 / 17 (32768); 256 experts, all
+// local: 24576 16 against 24. One workgroup for all experts had taken 16 / 17 at 8192 and 27 / 32 at
+// 16384.
+constexpr int kExpertMaxTasks = 24 * kExpertThreads;  // P = 24 passes a wave
 constexpr int kChunkThreads = 1024;
 constexpr int kChunkWaves = kChunkThreads / kWave;
 static_assert(kMaxExperts <= kChunkThreads, "the chunk-count reduction needs a thread per expert");
@@ -138,38 +145,121 @@ __device__ __forceinline__ void zero_sched(const RouteArgs& a) {
     for (int i = threadIdx.x; i < a.zero_count; i += blockDim.x) a.zero_ints[i] = 0;
 }
 
-__global__ __launch_bounds__(kSmallThreads) void route_small_kernel(RouteArgs a) {
+// One launch, a workgroup an expert and one more: workgroup e reads all the tasks, each of its 16
+// waves a contiguous range that stays in registers (up to P passes of 64 tasks), and counts with two
+// ballots a pass the tasks of lower experts (its row offset) and its own (the waves' bases); then
+// its own tasks' lanes write their rows. The last workgroup counts every expert, marks the tasks
+// without one and publishes counts, offsets, stats and meta. No workgroup waits for another.
+//
+// kBatch passes of the wave from task `begin` on, 32-bit task numbers: the experts, or -1.
+template <typename Id>
+__device__ __forceinline__ void expert_load(const RouteArgs& a, const Id* idx, int begin, int end, int* ev) {
+  Id id[kBatch];
+  float w[kBatch];
+#pragma unroll
+  for (int p = 0; p < kBatch; ++p) {
+    const uint32_t t = min(begin + p * kWave + lane_id(), end - 1);
+    id[p] = idx[t];
+    w[p] = a.topk_w[t];
+  }
+#pragma unroll
+  for (int p = 0; p < kBatch; ++p)
+    ev[p] = begin + p * kWave + lane_id() < end ? valid_expert(a, static_cast<int64_t>(id[p]), w[p]) : -1;
+}
+
+__device__ __forceinline__ void expert_load(const RouteArgs& a, int begin, int end, int* ev) {
+  if (a.idx_i64) expert_load(a, static_cast<const int64_t*>(a.topk_idx), begin, end, ev);
+  else expert_load(a, static_cast<const int32_t*>(a.topk_idx), begin, end, ev);
+}
+
+template <int P>
+__global__ __launch_bounds__(kExpertThreads) void route_expert_kernel(RouteArgs a) {
   zero_sched(a);  // (also when GEMM1 routes: the WIDE GEMM1 then returns at once, and the
                   // combine reads its zero-fill claim counter as zero)
   if (route_skipped(a)) return;
-  __shared__ int s_cnt[kSmallWaves][kSmallMaxExperts];
-  __shared__ int s_tot[kSmallMaxExperts];
-  __shared__ int s_off[kSmallMaxExperts + 1];
-  const int wave = threadIdx.x / kWave;
+  __shared__ int s_cnt[kExpertWaves][kExpertMaxExperts];
+  __shared__ int s_tot[kExpertMaxExperts];
+  __shared__ int s_off[kExpertMaxExperts + 1];
+  const int lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int E = a.num_experts;
-  const int64_t ntasks =
-      static_cast<int64_t>(effective_tokens(a.runtime_tokens, a.host_tokens)) * a.topk;
-  const int64_t per = ((ntasks + kSmallWaves - 1) / kSmallWaves + kWave - 1) / kWave * kWave;
-  const int64_t begin = wave * per;
-  const int64_t end = begin + per < ntasks ? begin + per : ntasks;
-  for (int i = threadIdx.x; i < kSmallWaves * E; i += kSmallThreads) s_cnt[i / E][i % E] = 0;
-  __syncthreads();
-  wave_route(a, begin, end, s_cnt[wave], [&]() {
+  const int e = blockIdx.x;
+  const int ntasks = effective_tokens(a.runtime_tokens, a.host_tokens) * a.topk;
+  const int per = ((ntasks + kExpertWaves - 1) / kExpertWaves + kWave - 1) / kWave * kWave;
+  const int begin = min(wave * per, ntasks);
+  const int end = min(begin + per, ntasks);
+  if (e == E) {
+    for (int i = threadIdx.x; i < kExpertWaves * E; i += kExpertThreads) s_cnt[i / E][i % E] = 0;
     __syncthreads();
-    for (int e = threadIdx.x; e < E; e += kSmallThreads) {
-      int run = 0;
-      for (int w = 0; w < kSmallWaves; ++w) {
-        const int c = s_cnt[w][e];
-        s_cnt[w][e] = run;
-        run += c;
+    // (LDS atomics into the wave's own row: integer sums, so the order of the lanes is no matter)
+    for (int b = begin; b < end; b += kBatch * kWave) {
+      int ev[kBatch];
+      expert_load(a, b, end, ev);
+#pragma unroll
+      for (int p = 0; p < kBatch; ++p) {
+        const int task = b + p * kWave + lane;
+        if (ev[p] >= 0) atomicAdd(&s_cnt[wave][ev[p]], 1);
+        else if (task < end) a.output_index[task] = -1;
       }
-      s_tot[e] = run;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < E; i += kExpertThreads) {
+      int run = 0;
+      for (int w = 0; w < kExpertWaves; ++w) run += s_cnt[w][i];
+      s_tot[i] = run;
     }
     __syncthreads();
     publish_offsets(a, s_tot, s_off, true);
-    for (int i = threadIdx.x; i < kSmallWaves * E; i += kSmallThreads) s_cnt[i / E][i % E] += s_off[i % E];
-    __syncthreads();
-  });
+    return;
+  }
+  int ev[P];
+  int lower = 0, own = 0;
+#pragma unroll
+  for (int p0 = 0; p0 < P; p0 += kBatch) {
+    if (begin + p0 * kWave >= end) break;
+    expert_load(a, begin + p0 * kWave, end, ev + p0);
+#pragma unroll
+    for (int p = p0; p < p0 + kBatch; ++p) {
+      own += __popcll(__ballot(ev[p] == e));
+      lower += __popcll(__ballot(static_cast<unsigned>(ev[p]) < static_cast<unsigned>(e)));  // (-1: not lower)
+    }
+  }
+  if (lane == 0) {
+    s_cnt[wave][0] = own;
+    s_cnt[wave][1] = lower;
+  }
+  if (a.given_counts != nullptr && wave == 0) {  // the caller's counts place the experts
+    int given = 0;
+    for (int i = lane; i < e; i += kWave) given += a.given_counts[i];
+    given = __shfl(wave_inclusive_sum(given), kWave - 1, kWave);
+    if (lane == 0) s_off[0] = given;
+  }
+  __syncthreads();
+  int row = a.given_counts != nullptr ? s_off[0] : 0;
+#pragma unroll
+  for (int w = 0; w < kExpertWaves; ++w)
+    row += (a.given_counts != nullptr ? 0 : s_cnt[w][1]) + (w < wave ? s_cnt[w][0] : 0);
+#pragma unroll
+  for (int p0 = 0; p0 < P; p0 += kBatch) {
+    if (begin + p0 * kWave >= end) break;
+#pragma unroll
+    for (int p = p0; p < p0 + kBatch; ++p) {
+      const uint64_t m = __ballot(ev[p] == e);
+      if (m == 0) continue;
+      if (ev[p] == e) {
+        const int task = begin + p * kWave + lane;
+        const int r = row + __popcll(m & lanes_below());
+        const bool kept = r < a.row_cap;
+        a.output_index[task] = kept ? r : -1;
+        if (kept) {
+          a.row_token[r] = task / a.topk;
+          if (a.row_weight != nullptr) a.row_weight[r] = a.topk_w[task];
+          if (a.m_indices != nullptr) a.m_indices[r] = e;
+        }
+      }
+      row += __popcll(m);
+    }
+  }
 }
 
 // The tasks of chunk `chunk` that wave `wave` of a chunk workgroup routes: the same split in
@@ -303,8 +393,10 @@ int64_t route_chunk_tasks(int64_t ntasks) {
 
 hipError_t launch_route(const RouteArgs& a, int64_t max_tasks, hipStream_t stream) {
   if (max_tasks <= 0) return hipSuccess;
-  if (max_tasks <= kSmallWaves * kRouteChunk && a.num_experts <= kSmallMaxExperts) {
-    return launch_kernel(route_small_kernel, dim3(1), dim3(kSmallThreads), 0, stream, a);
+  if (max_tasks <= kExpertMaxTasks && a.num_experts <= kExpertMaxExperts) {
+    const dim3 grid(static_cast<unsigned>(a.num_experts + 1)), block(kExpertThreads);
+    if (max_tasks <= 16 * kExpertThreads) return launch_kernel(route_expert_kernel<16>, grid, block, 0, stream, a);
+    return launch_kernel(route_expert_kernel<24>, grid, block, 0, stream, a);
   }
   const int64_t chunk = route_chunk_tasks(max_tasks);
   const int64_t chunks = (max_tasks + chunk - 1) / chunk;

@@ -15,7 +15,7 @@ namespace mmoe {
 
 // Expert of a task (or -1), from already-loaded id and weight.
 __device__ __forceinline__ int valid_expert(const RouteArgs& a, int64_t e, float w) {
-  if (e < 0 || e >= a.num_experts) return -1;
+  if (static_cast<uint64_t>(e) >= static_cast<uint64_t>(a.num_experts)) return -1;
   if (a.check_weight && w == 0.0f) return -1;
   return static_cast<int>(e);
 }

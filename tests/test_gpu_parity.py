@@ -132,6 +132,10 @@ ROUTE_CASES = {
     # chunks over 256 experts
     "chunks_ragged": (2731, 32, 6, 256),
     "chunks_e256": (4096, 256, 8, None),
+    # the workgroup-an-expert kernel's two sizes and the chunk kernels after them, 64 tasks short
+    # of and just past each limit (16,384 and 24,576 tasks); 256 and 3 experts
+    "expert_16k": (2720, 32, 6, 256), "expert_24k": (4096, 32, 6, None), "past_24k": (4097, 32, 6, 256),
+    "expert_e256": (3000, 256, 8, None), "expert_e3": (5000, 3, 2, None),
 }
 
 
@@ -1304,6 +1308,34 @@ def test_deepep_pre_post_process(mm, cuda, ids_dtype):
                 v = v * w[ok, j].view(-1, 1)
             acc[ok] += v
         assert torch.equal(y.cpu(), acc.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("s,slack", [(2000, 0), (5500, 3)])
+def test_deepep_preprocess_given_counts(mm, cuda, s, slack):
+    """The caller's counts place the experts (8 x 2000 and 8 x 5500 tasks: a workgroup an expert, the
+    chunk kernels): with counts above the tasks' own the rows left over read weight 0 and expert -1."""
+    e, k, hdim = 8, 8, 256
+    gen = torch.Generator().manual_seed(s)
+    x_fp8, x_sf = O.cast_to_fp8_channelwise(torch.randn((s, hdim), generator=gen).to(torch.bfloat16))
+    idx = torch.randint(-1, e, (s, k), generator=gen)
+    w = torch.rand((s, k), generator=gen)
+    ref = O.route(idx, torch.ones_like(w), e)
+    counts = torch.from_numpy(ref.counts).to(torch.int32) + slack
+    rows = int(counts.sum())
+    log(f"preprocess with given counts S={s} slack={slack}")
+    gx, gs, rw, mi, oi = mm.deepep_deepgemm_preprocess_channelwise(
+        x_fp8.to(cuda), x_sf.to(cuda), idx.to(cuda), w.to(cuda), counts.to(cuda), rows)
+    torch.cuda.synchronize()
+    shift = np.arange(e) * slack  # an expert's rows start `slack` later for each expert before it
+    row = np.arange(ref.num_rows) + shift[np.asarray(ref.m_indices)]
+    want = np.where(ref.output_index >= 0, row[np.maximum(ref.output_index, 0)], -1)
+    assert np.array_equal(oi.cpu().numpy(), want)
+    exp_mi, exp_w = np.full(rows, -1, np.int32), np.zeros(rows, np.float32)
+    exp_mi[row] = ref.m_indices
+    exp_w[row] = w.reshape(-1).numpy()[np.asarray(ref.row_token).astype(np.int64) * k + ref.row_slot]
+    assert np.array_equal(mi.cpu().numpy(), exp_mi) and np.array_equal(rw.cpu().numpy(), exp_w)
+    tok = torch.from_numpy(np.asarray(ref.row_token)).long()
+    assert torch.equal(gx[torch.from_numpy(row).to(cuda)].cpu().view(torch.uint8), x_fp8[tok].view(torch.uint8))
 
 
 def test_api_flag_and_tensor_errors(mm, cuda, monkeypatch):
