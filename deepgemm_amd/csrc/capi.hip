@@ -603,7 +603,13 @@ int mmoe_deepep_preprocess_channelwise(void* grouped_x, float* grouped_x_scale,
   if (workspace_bytes < need) return MMOE_ERR_SCRATCH_SMALL;
   if (hidden <= 0) return MMOE_ERR_HIDDEN_SIZES;
   const int64_t tasks = static_cast<int64_t>(recv_rows) * topk;
-  if (tasks == 0) return MMOE_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  // rows without a task: weight 0 and expert -1 (the routing writes output_index for every task)
+  if (tasks == 0)
+    return route_weights == nullptr || m_indices == nullptr ||
+                   mmoe::launch_clear_rows(route_weights, m_indices, total_rows, s) == hipSuccess
+               ? MMOE_OK
+               : MMOE_ERR_HIP;
   if (grouped_x == nullptr || grouped_x_scale == nullptr || route_weights == nullptr ||
       m_indices == nullptr || output_index == nullptr || recv_x == nullptr ||
       recv_x_scale == nullptr || recv_topk_ids == nullptr || recv_topk_weights == nullptr ||
@@ -636,7 +642,7 @@ int mmoe_deepep_preprocess_channelwise(void* grouped_x, float* grouped_x_scale,
   r.output_index = output_index;
   r.row_weight = route_weights;
   r.m_indices = m_indices;
-  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (mmoe::launch_clear_rows(route_weights, m_indices, total_rows, s) != hipSuccess) return MMOE_ERR_HIP;
   if (mmoe::launch_route(r, tasks, s) != hipSuccess) return MMOE_ERR_HIP;
   if (mmoe::launch_gather_tasks(static_cast<uint8_t*>(grouped_x), grouped_x_scale,
                                 static_cast<const uint8_t*>(recv_x), recv_x_scale, output_index,

@@ -306,6 +306,14 @@ __global__ __launch_bounds__(kEltThreads) void gather_tasks_kernel(uint8_t* gx, 
   }
 }
 
+// The rows that the routing may leave out (counts above the tasks' own): weight 0, expert -1.
+__global__ __launch_bounds__(kEltThreads) void clear_rows_kernel(float* row_weight, int32_t* m_indices, int rows) {
+  for (int r = blockIdx.x * kEltThreads + threadIdx.x; r < rows; r += gridDim.x * kEltThreads) {
+    row_weight[r] = 0.0f;
+    m_indices[r] = -1;
+  }
+}
+
 // ---------------------------------------------------------------- channelwise cast
 // scale = max(amax, 1e-4) / 448 and the codes e4m3(clip(x / scale)) of rows of bf16. Every value is
 // read from memory once: it stays in registers between the row's maximum and its codes.
@@ -524,6 +532,12 @@ hipError_t launch_combine(const CombineArgs& c, int num_cus, hipStream_t stream)
     const unsigned grid = grid_for(c.host_tokens, 1, static_cast<int64_t>(num_cus) * 16);
     return launch_kernel(combine_scalar_kernel, dim3(grid), dim3(kEltThreads), 0, stream, c);
   }
+}
+
+hipError_t launch_clear_rows(float* row_weight, int32_t* m_indices, int rows, hipStream_t stream) {
+  if (rows <= 0) return hipSuccess;
+  return launch_kernel(clear_rows_kernel, dim3(grid_for(rows, kEltThreads, 1024)), dim3(kEltThreads), 0,
+                       stream, row_weight, m_indices, rows);
 }
 
 hipError_t launch_gather_tasks(uint8_t* grouped_x, float* grouped_scale, const uint8_t* x,

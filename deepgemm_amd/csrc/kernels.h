@@ -245,6 +245,9 @@ struct PipeArgs {
 bool decode_pipeline_supported(const GemmArgs& g1, const GemmArgs& g2, int num_cus);
 hipError_t launch_decode_pipeline(const PipeArgs& p, int num_cus, hipStream_t stream);
 
+// row_weight[r] = 0 and m_indices[r] = -1 for r < rows (the preprocess, before the routing).
+hipError_t launch_clear_rows(float* row_weight, int32_t* m_indices, int rows, hipStream_t stream);
+
 // For every task (token t, slot s) with row = output_index[t*K+s] >= 0:
 // grouped_x[row] = x[t], grouped_scale[row] = x_sf[t].
 hipError_t launch_gather_tasks(uint8_t* grouped_x, float* grouped_scale, const uint8_t* x,

@@ -77,7 +77,9 @@ def _is_current_stream_capturing() -> bool:
 
 
 def _stream_handle() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream of the current device (the raw handle: a torch.cuda.Stream object for it
+    costs 3 us a call, this 0.3)."""
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -395,9 +397,10 @@ def deepep_deepgemm_preprocess_channelwise(recv_x: torch.Tensor, recv_x_scale: t
     dev = recv_x.device
     grouped_x = torch.empty((rows, hidden), dtype=torch.float8_e4m3fn, device=dev)
     grouped_x_scale = torch.empty((rows,), dtype=torch.float32, device=dev)
-    route_weights = torch.zeros((rows,), dtype=torch.float32, device=dev)
-    m_indices = torch.full((rows,), -1, dtype=torch.int32, device=dev)
-    output_index = torch.full((recv_rows, topk), -1, dtype=torch.int32, device=dev)
+    # filled by the library: rows without a task get weight 0 and expert -1, every task its row or -1
+    route_weights = torch.empty((rows,), dtype=torch.float32, device=dev)
+    m_indices = torch.empty((rows,), dtype=torch.int32, device=dev)
+    output_index = torch.empty((recv_rows, topk), dtype=torch.int32, device=dev)
     lib = _capi.load()
     ws_bytes = ctypes.c_int64()
     _capi.check(lib.mmoe_deepep_preprocess_workspace_bytes(recv_rows, topk, num_experts, rows,

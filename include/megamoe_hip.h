@@ -252,7 +252,8 @@ int mmoe_route(const mmoe_forward_args* args, void* stream);
 /* deepep_deepgemm_preprocess_channelwise, csrc/apis/mega_dcu.hpp:222-292 with
  * csrc/kernels/mega_moe_baseline_hip.cu:37-96. Expert-contiguous scatter of received rows.
  * Rows of an expert are in ascending (token, slot) order (deterministic). Outputs sized
- * [total_rows, ...]; the caller pre-fills route_weights=0, m_indices=-1 like the reference.
+ * [total_rows, ...]; rows without a task get route_weights 0 and m_indices -1 (the reference's
+ * caller pre-fills those).
  * topk_ids are int64 when topk_ids_i64 != 0 else int32. `workspace` is device scratch of at
  * least mmoe_deepep_preprocess_workspace_bytes() bytes (the reference's expert_start_loc). */
 int mmoe_deepep_preprocess_workspace_bytes(int recv_rows, int topk, int num_experts,

@@ -1338,6 +1338,19 @@ def test_deepep_preprocess_given_counts(mm, cuda, s, slack):
     assert torch.equal(gx[torch.from_numpy(row).to(cuda)].cpu().view(torch.uint8), x_fp8[tok].view(torch.uint8))
 
 
+def test_deepep_preprocess_no_tokens(mm, cuda):
+    """No received tokens: no rows are routed, and the rows asked for read weight 0 and expert -1."""
+    e, k, hdim = 8, 4, 256
+    log("preprocess without tokens")
+    for rows in (0, 700):
+        gx, gs, rw, mi, oi = mm.deepep_deepgemm_preprocess_channelwise(
+            torch.empty((0, hdim), dtype=torch.float8_e4m3fn, device=cuda), torch.empty((0,), device=cuda),
+            torch.empty((0, k), dtype=torch.int64, device=cuda), torch.empty((0, k), device=cuda),
+            torch.zeros((e,), dtype=torch.int32, device=cuda), rows)
+        assert gx.shape == (max(rows, 1), hdim) and oi.shape == (0, k)
+        assert torch.all(rw == 0) and torch.all(mi == -1)
+
+
 def test_api_flag_and_tensor_errors(mm, cuda, monkeypatch):
     """The reference's flag and tensor checks raise the same exception types and messages
     (megamoe/__init__.py:343-410, csrc/apis/mega_dcu.hpp:355-433, large_opt.py:381, :526,
