@@ -14,7 +14,7 @@
 // counts become per-wave bases through LDS prefix sums.
 //
 // Two launch shapes, both integer work bound by the topk tables' reads and their latency:
-//   * up to 24576 tasks: one launch with a workgroup for each expert, which ranks that expert's tasks;
+//   * up to 16384 tasks: one launch with a workgroup for each expert, which ranks that expert's tasks;
 //   * more: a count kernel (one workgroup per chunk, LDS histogram) and a scatter kernel
 //     (one workgroup per chunk) that rebuilds the expert offsets and its chunk base from the
 //     per-chunk counts itself, so no grid-wide barrier or separate scan launch is needed.
@@ -29,16 +29,15 @@ constexpr int kExpertThreads = 1024;
 constexpr int kExpertWaves = kExpertThreads / kWave;
 constexpr int kExpertMaxExperts = 256;
 // Tasks up to which a workgroup an expert routes: it reads all of them, so its time grows with their
-// number, while the chunk kernels' two launches have a floor of 17 us. 32 experts, us (one of 8 slots
-// local / all of them local): 8192 tasks 5.6 / 7.2, 16384 8.3 / 11.6, 24576 10.4 / 16.1, 32768
-// 12.6 / 19.9, against the chunk kernels' 17 / 17 (24576) and 17 / 17 (32768); 256 experts, all
-// local: 24576 16 against 24. One workgroup for all experts had taken 16 / 17 at 8192 and 27 / 32 at
-// 16384.
-constexpr int kExpertMaxTasks = 24 * kExpertThreads;  // P = 24 passes a wave
+// number, while the chunk kernels' two launches have a floor of 10.5 us. 32 experts, us (one of 8
+// slots local / all of them local): 8192 tasks 5.6 / 7.2, 16384 8.3 / 11.6, 24576 10.4 / 16.1, against
+// the chunk kernels' 10.5 / 11 at 24576. One workgroup for all experts had taken 16 / 17 at 8192 and
+// 27 / 32 at 16384.
+constexpr int kExpertPasses = 16;  // of a wave
+constexpr int kExpertMaxTasks = kExpertPasses * kExpertThreads;
 constexpr int kChunkThreads = 1024;
 constexpr int kChunkWaves = kChunkThreads / kWave;
 static_assert(kMaxExperts <= kChunkThreads, "the chunk-count reduction needs a thread per expert");
-static_assert(2 * kChunkThreads <= kChunkWaves * kMaxExperts, "partial sums fit in s_wbase");
 static_assert(kChunkWaves == kRouteWaves, "per-wave counts of a chunk in the workspace");
 
 // Assigns rows to one 64-task pass in task order; base[e] is this wave's running base.
@@ -72,26 +71,35 @@ __device__ void wave_count_range(const RouteArgs& a, int64_t begin, int64_t end,
   for (int64_t b = begin; b < end; b += kBatch * kWave) {
     wave_load<kBatch>(a, b, end, ev, wv);
 #pragma unroll
-    for (int p = 0; p < kBatch; ++p) wave_count_pass(ev[p], id_bits, row);
+    for (int p = 0; p < kBatch; ++p) {
+      if (b + p * kWave >= end) break;  // (a chunk of 1024 tasks has one pass a wave)
+      wave_count_pass(ev[p], id_bits, row);
+    }
   }
 }
 
-// counted: the count rows hold this range's counts already (the count kernel's).
-template <class Gap>
-__device__ void wave_route(const RouteArgs& a, int64_t begin, int64_t end, int* row,
-                           Gap phase_gap, bool counted = false) {
+// A wave's first kBatch passes of tasks, loaded ahead.
+struct WaveTasks {
   int ev[kBatch];
   float wv[kBatch];
+};
+
+// counted: the count rows hold this range's counts already (the count kernel's). `t` holds the
+// range's first batch.
+template <class Gap>
+__device__ void wave_route(const RouteArgs& a, int64_t begin, int64_t end, int* row, WaveTasks& t,
+                           Gap phase_gap, bool counted) {
   const int id_bits = expert_id_bits(a.num_experts);
   if (!counted) wave_count_range(a, begin, end, row);
   phase_gap();
   const int lane = lane_id();
   for (int64_t b = begin; b < end; b += kBatch * kWave) {
-    wave_load<kBatch>(a, b, end, ev, wv);
+    if (b > begin) wave_load<kBatch>(a, b, end, t.ev, t.wv);
 #pragma unroll
     for (int p = 0; p < kBatch; ++p) {
+      if (b + p * kWave >= end) break;
       const int64_t task = b + p * kWave + lane;
-      wave_scatter_pass(a, task, task < end, ev[p], wv[p], id_bits, row);
+      wave_scatter_pass(a, task, task < end, t.ev[p], t.wv[p], id_bits, row);
     }
   }
 }
@@ -146,7 +154,7 @@ __device__ __forceinline__ void zero_sched(const RouteArgs& a) {
 }
 
 // One launch, a workgroup an expert and one more: workgroup e reads all the tasks, each of its 16
-// waves a contiguous range that stays in registers (up to P passes of 64 tasks), and counts with two
+// waves a contiguous range that stays in registers (up to 16 passes of 64 tasks), and counts with two
 // ballots a pass the tasks of lower experts (its row offset) and its own (the waves' bases); then
 // its own tasks' lanes write their rows. The last workgroup counts every expert, marks the tasks
 // without one and publishes counts, offsets, stats and meta. No workgroup waits for another.
@@ -172,7 +180,6 @@ __device__ __forceinline__ void expert_load(const RouteArgs& a, int begin, int e
   else expert_load(a, static_cast<const int32_t*>(a.topk_idx), begin, end, ev);
 }
 
-template <int P>
 __global__ __launch_bounds__(kExpertThreads) void route_expert_kernel(RouteArgs a) {
   zero_sched(a);  // (also when GEMM1 routes: the WIDE GEMM1 then returns at once, and the
                   // combine reads its zero-fill claim counter as zero)
@@ -212,6 +219,7 @@ __global__ __launch_bounds__(kExpertThreads) void route_expert_kernel(RouteArgs 
     publish_offsets(a, s_tot, s_off, true);
     return;
   }
+  constexpr int P = kExpertPasses;
   int ev[P];
   int lower = 0, own = 0;
 #pragma unroll
@@ -313,18 +321,31 @@ __global__ __launch_bounds__(kChunkThreads) void route_chunk_scatter_kernel(Rout
   __shared__ int s_tot[kMaxExperts];
   __shared__ int s_off[kMaxExperts + 1];
   __shared__ int s_cbase[kMaxExperts];
+  __shared__ int s_part[2 * kChunkThreads];  // 2 * groups * E <= 2 * 1024
   const int tid = threadIdx.x;
   const int wave = tid / kWave;
   const int E = a.num_experts;
   const int chunk = blockIdx.x;
+  // Every load that does not wait for another goes out first: this wave's tasks, the count kernel's
+  // per-wave counts of this chunk (same task split; null: count again) and every chunk's counts.
+  // Side by side, and without the passes past a wave's range, they took the two launches from 17.2 to
+  // 10.9 us at 49,152 tasks and from 21.0 to 18.9 at 1.57 M (32 of 256 experts).
+  const int64_t ntasks =
+      static_cast<int64_t>(effective_tokens(a.runtime_tokens, a.host_tokens)) * a.topk;
+  const WaveRange wr = chunk_wave_range(ntasks, chunk, chunk_tasks, wave);
+  WaveTasks tasks;
+  wave_load<kBatch>(a, wr.begin, wr.end, tasks.ev, tasks.wv);
+  const bool counted = a.wave_counts != nullptr;
+  const int32_t* wsrc = counted ? a.wave_counts + static_cast<int64_t>(chunk) * kChunkWaves * E : nullptr;
+  for (int i = tid; i < kChunkWaves * E; i += kChunkThreads) s_wbase[i / E][i % E] = counted ? wsrc[i] : 0;
   // Totals and this chunk's base per expert, from every chunk's counts. Thread t sums the
   // chunks g, g + G, g + 2G, ... of expert e = t % E (g = t / E, G = 1024 / E groups), so all
   // threads load at once (consecutive threads, consecutive experts of a chunk row); the G
-  // partial sums of an expert then meet in LDS (s_wbase as scratch, before its own use).
+  // partial sums of an expert then meet in LDS.
   {
     const int groups = kChunkThreads / E;  // >= 1: E <= kMaxExperts == kChunkThreads
-    int* s_ptot = &s_wbase[0][0];
-    int* s_pbase = s_ptot + groups * E;   // 2 * groups * E <= 2 * 1024 ints of s_wbase
+    int* s_ptot = s_part;
+    int* s_pbase = s_part + groups * E;
     if (tid < groups * E) {
       const int e = tid % E, g = tid / E;
       int tot = 0, base = 0;
@@ -360,15 +381,7 @@ __global__ __launch_bounds__(kChunkThreads) void route_chunk_scatter_kernel(Rout
     __syncthreads();
   }
   publish_offsets(a, s_tot, s_off, chunk == 0);
-  const int64_t ntasks =
-      static_cast<int64_t>(effective_tokens(a.runtime_tokens, a.host_tokens)) * a.topk;
-  const WaveRange wr = chunk_wave_range(ntasks, chunk, chunk_tasks, wave);
-  // the count kernel's per-wave counts of this chunk (same task split), else count again
-  const bool counted = a.wave_counts != nullptr;
-  const int32_t* wsrc = counted ? a.wave_counts + static_cast<int64_t>(chunk) * kChunkWaves * E : nullptr;
-  for (int i = tid; i < kChunkWaves * E; i += kChunkThreads) s_wbase[i / E][i % E] = counted ? wsrc[i] : 0;
-  __syncthreads();
-  wave_route(a, wr.begin, wr.end, s_wbase[wave], [&]() {
+  wave_route(a, wr.begin, wr.end, s_wbase[wave], tasks, [&]() {
     __syncthreads();
     for (int e = tid; e < E; e += kChunkThreads) {
       int run = s_off[e] + s_cbase[e];
@@ -394,9 +407,8 @@ int64_t route_chunk_tasks(int64_t ntasks) {
 hipError_t launch_route(const RouteArgs& a, int64_t max_tasks, hipStream_t stream) {
   if (max_tasks <= 0) return hipSuccess;
   if (max_tasks <= kExpertMaxTasks && a.num_experts <= kExpertMaxExperts) {
-    const dim3 grid(static_cast<unsigned>(a.num_experts + 1)), block(kExpertThreads);
-    if (max_tasks <= 16 * kExpertThreads) return launch_kernel(route_expert_kernel<16>, grid, block, 0, stream, a);
-    return launch_kernel(route_expert_kernel<24>, grid, block, 0, stream, a);
+    return launch_kernel(route_expert_kernel, dim3(static_cast<unsigned>(a.num_experts + 1)),
+                         dim3(kExpertThreads), 0, stream, a);
   }
   const int64_t chunk = route_chunk_tasks(max_tasks);
   const int64_t chunks = (max_tasks + chunk - 1) / chunk;

@@ -132,10 +132,10 @@ ROUTE_CASES = {
     # chunks over 256 experts
     "chunks_ragged": (2731, 32, 6, 256),
     "chunks_e256": (4096, 256, 8, None),
-    # the workgroup-an-expert kernel's two sizes and the chunk kernels after them, 64 tasks short
-    # of and just past each limit (16,384 and 24,576 tasks); 256 and 3 experts
-    "expert_16k": (2720, 32, 6, 256), "expert_24k": (4096, 32, 6, None), "past_24k": (4097, 32, 6, 256),
-    "expert_e256": (3000, 256, 8, None), "expert_e3": (5000, 3, 2, None),
+    # the workgroup-an-expert kernel at its limit (16,384 tasks, also over 256 experts) and at the
+    # smallest size with an empty wave, with 3 experts; the chunk kernels at 24,576 and more tasks
+    "expert_16k": (4096, 32, 4, 256), "expert_e256": (2048, 256, 8, None), "expert_e3": (480, 3, 2, None),
+    "chunks_24k": (4096, 32, 6, None), "chunks_24582": (4097, 32, 6, 256),
 }
 
 
