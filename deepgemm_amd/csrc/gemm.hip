@@ -66,6 +66,7 @@ constexpr int kStreamDepth = 4;     // 64-k weight steps in flight per wave
 constexpr int kAChunk = 65536;      // bytes of one A chunk buffer (32*MT rows x 2048/MT k)
 constexpr int kALoads = kAChunk / 1024 / kGemmWaves;  // 16-byte A loads per lane per chunk
 constexpr int kNarrowDepth = 8;     // weight steps in flight of a narrow item's waves
+constexpr int kAChunk4 = kAChunk / 256;  // k-bytes of a chunk of 128 rows in half a buffer
 // TILE engine: 256 x 256 output tile, BK = 128, the 8 waves as 2 (M) x 4 (N), each wave 128
 // rows x 64 columns (4 x 2 MFMA tiles of 32 x 32)
 constexpr int kTileBM = 256, kTileBN = 256, kTileBK = 128;
@@ -1399,7 +1400,9 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs 
         rs = RowSrc{s_tok, s_rw, row0};
       }
       if (mrows > 64) {
-        stream_tile<kGather, kSwiglu, 4, 2>(g, rs, e, row0, mrows, nb, g.kc[2], smem, s_tt);
+        if (!kAnyK || g.ring[2] == 4)
+          stream_tile<kGather, kSwiglu, 4, 4, false, false, false, false, false, kALoads / 2>(g, rs, e, row0, mrows, nb, kAChunk4, smem, s_tt);
+        else if (kAnyK) stream_tile<kGather, kSwiglu, 4, 2>(g, rs, e, row0, mrows, nb, g.kc[2], smem, s_tt);
       } else if (mrows > 32) {
         if (!kAnyK || g.ring[1] == 4) stream_tile<kGather, kSwiglu, 2, 4>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
         else if (kAnyK) stream_tile<kGather, kSwiglu, 2, 2>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
@@ -1851,7 +1854,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
         if (kSmall && waves < kGemmWaves)
           stream_tile<true, true, 1, kNarrowDepth, true, false, true, true, true, kALoads / 2>(q.g1, rs, e, row0, mrows, nb, q.narrow_kc1, smem, s_tt, rank_rows, waves);
         else if (!kSmall && mrows > 64)
-          stream_tile<true, true, 4, 2, true, false, true, true, false, kALoads / 2>(q.g1, rs, e, row0, mrows, nb, q.half_kc4, smem, s_tt, rank_rows);
+          stream_tile<true, true, 4, 2, true, false, true, true, false, kALoads / 2>(q.g1, rs, e, row0, mrows, nb, kAChunk4, smem, s_tt, rank_rows);
         else if (!kSmall && mrows > 32)
           stream_tile<true, true, 2, kStreamDepth, true, false, true, true>(q.g1, rs, e, row0, mrows, nb, q.g1.kc[1], smem, s_tt, rank_rows);
         else
@@ -2102,22 +2105,26 @@ int stream_chunk(int k, int cap, int steps) {
 
 // The STREAM engine's chunks of K for 1, 2 and 4 row tiles: as long as the LDS buffers allow, so that
 // the workgroup's barriers are few, with a ring of 4 weight steps unless a ring of 2 makes a chunk at
-// least twice as long (K not a multiple of 256: 640 = 10 steps). Four row tiles always have 2.
+// least twice as long (K not a multiple of 256: 640 = 10 steps). Beside the accumulators of 4 row
+// tiles a ring of 4 leaves registers for half the A loads only, so chunks of 256 in half the buffers:
+// 2715 rows of 32 experts 181.5 -> 177 us a layer against a ring of 2 and chunks of 512.
 void set_stream_chunks(GemmArgs* g) {
-  for (int i = 0; i < 3; ++i) {
+  for (int i = 0; i < 2; ++i) {
     const int cap = kAChunk / 32 >> i;
-    const int four = i < 2 ? stream_chunk(g->k, cap, kStreamDepth) : 0;
+    const int four = stream_chunk(g->k, cap, kStreamDepth);
     const int two = stream_chunk(g->k, cap, 2);
     g->ring[i] = 2 * four > two ? kStreamDepth : 2;
     g->kc[i] = 2 * four > two ? four : two;
   }
+  g->ring[2] = g->k % kAChunk4 == 0 ? kStreamDepth : 2;
+  g->kc[2] = g->k % kAChunk4 == 0 ? kAChunk4 : stream_chunk(g->k, kAChunk / 128, 2);
 }
 
 template <bool kGather, bool kSwiglu>
 hipError_t launch_engines(const GemmArgs& args, int max_rows, int num_cus, hipStream_t stream) {
   GemmArgs g = args;
   set_stream_chunks(&g);
-  return g.ring[0] == 4 && g.ring[1] == 4
+  return g.ring[0] == 4 && g.ring[1] == 4 && g.ring[2] == 4
              ? launch_engines_k<kGather, kSwiglu, false>(g, max_rows, num_cus, stream)
              : launch_engines_k<kGather, kSwiglu, true>(g, max_rows, num_cus, stream);
 }
@@ -2214,7 +2221,6 @@ hipError_t launch_decode_pipeline(const PipeArgs& args, int num_cus, hipStream_t
   set_stream_chunks(&p.g1);
   set_stream_chunks(&p.g2);
   p.narrow_kc1 = stream_chunk(p.g1.k, kAChunk / 64, kNarrowDepth);
-  p.half_kc4 = stream_chunk(p.g1.k, kAChunk / 256, 2);
   return launch_kernel(small ? decode_pipeline_kernel<true> : decode_pipeline_kernel<false>,
                        dim3(static_cast<unsigned>(num_cus)), dim3(kGemmThreads), kSmemBytes, stream, p);
 }

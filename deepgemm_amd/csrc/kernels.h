@@ -237,10 +237,7 @@ struct PipeArgs {
                          // H % 8 == 0)
   int spin_limit;        // polls of a bounded wait: kPipeSpinLimit, or 0 to test the error path
                          // (every wait then gives up at once)
-  // GEMM1's k-bytes a chunk in narrow items, and in items of 4 row tiles (half A chunk buffers, so
-  // that the accumulators leave registers for the loads); set by the launch function
-  int narrow_kc1;
-  int half_kc4;
+  int narrow_kc1;        // GEMM1's k-bytes a chunk in narrow items (set by the launch function)
 };
 bool decode_pipeline_supported(const GemmArgs& g1, const GemmArgs& g2, int num_cus);
 hipError_t launch_decode_pipeline(const PipeArgs& p, int num_cus, hipStream_t stream);
