@@ -456,7 +456,9 @@ int mmoe_forward_stages(const mmoe_forward_args* a, int first_stage, int last_st
     p.direct_flag = direct_flag;
     p.pipe = at<int32_t>(ws, l.pipe_offset);
     p.spin_limit = (a->debug_flags & MMOE_DEBUG_NO_WAIT) != 0 ? 0 : mmoe::kPipeSpinLimit;
-    if (runs(MMOE_STAGE_COMBINE) && a->hidden % 8 == 0) {
+    // (the combine in the launch addresses the partial rows with 32-bit byte offsets)
+    const int64_t part_bytes = static_cast<int64_t>(a->num_tokens) * a->num_topk * a->hidden * 2;
+    if (runs(MMOE_STAGE_COMBINE) && a->hidden % 8 == 0 && part_bytes < int64_t{1} << 31) {
       p.y = static_cast<uint16_t*>(a->y);
       combined = true;
     }
