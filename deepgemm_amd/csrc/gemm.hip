@@ -1682,14 +1682,15 @@ __device__ void stage_rows_from_y(const PipeArgs& p, int row0, int mrows, int kc
   }
 }
 
-// The items [0, total) of one GEMM dealt to the XCDs in equal contiguous ranges. Wave 0 holds in one
-// register (`held`) the workgroup's next claim (lane 0) and what the XCDs' counters read when that
-// claim went out (XCD q's in lane kPeekLane + q).
+// The items of one GEMM, `units` pieces of `step` items, dealt to the XCDs in equal contiguous ranges of
+// whole pieces. Wave 0 holds in one register (`held`) the workgroup's next claim (lane 0) and what the
+// XCDs' counters read when that claim went out (XCD q's in lane kPeekLane + q).
 constexpr int kPeekLane = 8;
 struct PipeDeal {
   int32_t* claims;  // XCD x's counter at claims[x * kPipeLine]
-  int total;
-  __device__ __forceinline__ int begin(int x) const { return static_cast<int>(static_cast<int64_t>(total) * x / kPipeXcds); }
+  int units;
+  int step;
+  __device__ __forceinline__ int begin(int x) const { return static_cast<int>(static_cast<int64_t>(units) * x / kPipeXcds) * step; }
   __device__ __forceinline__ int size(int x) const { return begin(x + 1) - begin(x); }
   // wave 0: claims the next item of XCD x and peeks at all counters
   __device__ __forceinline__ int claim(int x) const {
@@ -1791,12 +1792,23 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
   const int G = __builtin_amdgcn_readfirstlane(too_many ? 0 : s_prefix1[E]);
   const int waves = Shape::units(G);
   const int n1 = g1.n / (kStreamUnit * waves), n2 = g2.n / (kStreamUnit * waves);
+  // Whole groups to an XCD, one group's items after the other's, when a last round of GEMM1 items keeps
+  // at most half of the CUs: the others go on to GEMM2 meanwhile, and the groups of the rounds before
+  // are complete then. Dealt item by item, a group's items can lie in two XCDs' ranges, and column block
+  // by column block an expert's groups end together: the first GEMM2 items then wait for the last round
+  // (1560, 1800 and 2040 Zipf rows: 198, 197 and 197 us; whole groups 184, 185 and 187). Above half, the even
+  // deal ends the last round earlier (2160, 2400 and 2640 rows: 199, 201 and 200 us; whole groups 204, 213
+  // and 217).
+  const int items1 = G * n1, last_round = items1 % static_cast<int>(gridDim.x);
+  const bool by_group = items1 > static_cast<int>(gridDim.x) && 2 * last_round <= static_cast<int>(gridDim.x) &&
+                        s_rows1 == Shape::kRows2;
   const float* task_w = reinterpret_cast<const float*>(smem);  // valid until the first item's loads
   bool first_item = true;
   for (int phase = 0; phase < 2; ++phase) {
     const bool gemm1 = phase == 0;
-    const PipeDeal deal{p.pipe + (gemm1 ? 0 : kPipeClaim2),
-                        gemm1 ? G * n1 : too_many ? 0 : __builtin_amdgcn_readfirstlane(s_prefix2[E]) * n2};
+    const int chunks = gemm1 ? G : too_many ? 0 : __builtin_amdgcn_readfirstlane(s_prefix2[E]);
+    const int blocks = gemm1 ? n1 : n2;
+    const PipeDeal deal{p.pipe + (gemm1 ? 0 : kPipeClaim2), by_group ? chunks : chunks * blocks, by_group ? blocks : 1};
     if (!gemm1) held = threadIdx.x == 0 ? s_claim2 : 0;
     int x = home;
     for (;;) {
@@ -1826,15 +1838,16 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
       if (threadIdx.x < kWave) held = deal.claim(x);  // the next claim, one item ahead
       const PipeArgs& q = item_args();
       // item t: an expert's items column block by column block, the chunks of a block next to each
-      // other, so that they run together and read its weights from HBM once
+      // other, so that they run together and read its weights from HBM once (by_group: chunk by chunk)
       const int t = deal.begin(x) + c;
       const int* s_prefix = gemm1 ? s_prefix1 : s_prefix2;
       const int per = gemm1 ? n1 : n2;
       const int e = expert_of_item(s_prefix, E, t / per);
       const int first = __builtin_amdgcn_readfirstlane(s_prefix[e]);
       const int nch = __builtin_amdgcn_readfirstlane(s_prefix[e + 1]) - first;
-      const int nb = (t - first * per) / nch;
-      const int ch = t - first * per - nb * nch;
+      const int local = t - first * per;
+      const int nb = by_group ? local % per : local / nch;
+      const int ch = by_group ? local / per : local - nb * nch;
       const int rows1 = __builtin_amdgcn_readfirstlane(s_rows1);
       const int rows = gemm1 ? rows1 : Shape::kRows2;
       const int r0 = ch * rows;

@@ -785,6 +785,8 @@ def test_decode_pipeline_many_experts(mm, cuda, e, s, g):
 PIPE_CASES = {
     "one_token": (1, None), "few": (8, 256), "some": (24, 256), "many": (53, None), "skewed": (48, "zipf"),
     "large_kernel": (54, 256), "groups_128": (420, None), "groups_64": (341, "zipf"),
+    # a last round of items below and above half of the CUs: whole groups to an XCD, items dealt evenly
+    "whole_groups": (270, "zipf"), "even_items": (440, "zipf"),
 }
 
 
@@ -811,6 +813,9 @@ def test_decode_pipeline_item_shapes(mm, cuda, full_weights, case):
         assert tr.routing.counts.max() > 32
     if case == "groups_128":
         assert tr.routing.counts.max() > 64
+    if case in ("whole_groups", "even_items"):  # 8 column blocks a group, 256 CUs
+        groups = int(sum(-(-int(n) // 64) for n in tr.routing.counts))
+        assert 8 * groups > 256 and (8 * groups % 256 <= 128) == (case == "whole_groups")
     _stage_checks(buf, tr, s)
     _combine_bitwise(mm, buf, y, l1, l2, s, None)
     assert O.calc_diff(y.cpu(), tr.y) <= CALC_DIFF_BAR
@@ -1308,6 +1313,28 @@ def test_deepep_pre_post_process(mm, cuda, ids_dtype):
                 v = v * w[ok, j].view(-1, 1)
             acc[ok] += v
         assert torch.equal(y.cpu(), acc.to(torch.bfloat16))
+
+
+def test_decode_pipeline_small_whole_groups(mm, cuda):
+    """The small kernel with more than a round of items (40 experts with rows, 8 column blocks in GEMM1
+    and 2 in GEMM2): whole groups to an XCD, in both GEMMs."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the decode pipeline runs on the whole 256-CU MI355X only")
+    e, k, s, hdim, inter = 40, 8, 40, 1024, 2048
+    log("small pipeline, whole groups")
+    x_fp8, x_sf, idx, w = make_tokens(s, hdim, e, k, seed=40)
+    l1, l2 = make_weights_gpu(e, hdim, inter, seed=41, mm=mm)
+    buf = mm.get_symm_buffer_for_mega_moe(None, e, s, k, hdim, inter)
+    buf.scratch_view("pmax").fill_(-1.0)
+    y = run_layer(mm, buf, x_fp8, x_sf, idx, w, l1, l2)
+    torch.cuda.synchronize()
+    tr = O.mega_moe_forward(x_fp8, x_sf, idx, w, *cpu_weights(l1, l2))
+    groups = int(sum(-(-int(n) // 32) for n in tr.routing.counts))
+    assert 32 < groups <= 48
+    assert bool((buf.scratch_view("pmax")[:tr.routing.num_rows] >= 0).all()), "the pipeline ran"
+    _stage_checks(buf, tr, s)
+    _combine_bitwise(mm, buf, y, l1, l2, s, None)
+    assert O.calc_diff(y.cpu(), tr.y) <= CALC_DIFF_BAR
 
 
 @pytest.mark.parametrize("s,slack", [(2000, 0), (5500, 3)])
