@@ -1435,8 +1435,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs 
 // invalidates its CU's L1 and requantizes the group's rows straight into its LDS A buffers (the
 // requant kernel's arithmetic, so the same bits; the group's first GEMM2 item also writes act
 // and amax out). It reads the rows through its own L2, which holds none of their lines: nothing in
-// this launch reads a row's line before the row's group is complete (a row is whole lines). The
-// maxima, whose lines two groups can share, it reads device-coherent. A workgroup starts on GEMM2
+// this launch reads a row's line before the row's group is complete (a row is whole lines:
+// decode_pipeline_supported). The maxima, whose lines two groups can share, it reads device-coherent. A workgroup starts on GEMM2
 // items only when every GEMM1 item is claimed, and a GEMM1 item waits on nothing, so every wait
 // ends, also when some XCDs have no workgroups; a wait is also bounded (kPipeSpinLimit polls), and
 // one that runs out is counted (the launch's last workgroup leaves the count in meta[3], the call's
@@ -2205,6 +2205,9 @@ static bool pipe_small(const GemmArgs& g1) {
 // Past the small kernel's tasks it also wants whole A chunks in both GEMMs: at H = 7168 or I = 1536
 // the separate launches are as fast there with few rows an expert (I = 1536, 512 tokens of 128
 // experts: 120 us against 116) and faster with many (R = 2139: 204 against 130).
+// And y in whole 128-byte lines (a caller's route_scratch can lie anywhere): a line that the last row
+// of one group shared with the first row of the next would come into an XCD's L2 with the first group's
+// rows, before the second group's are written. The separate launches take any other base.
 bool decode_pipeline_supported(const GemmArgs& g1, const GemmArgs& g2, int num_cus) {
   GemmArgs c1 = g1, c2 = g2;
   set_stream_chunks(&c1);
@@ -2212,7 +2215,7 @@ bool decode_pipeline_supported(const GemmArgs& g1, const GemmArgs& g2, int num_c
   const bool whole_chunks = g1.k % (kAChunk / 32) == 0 && g2.k == kAChunk / 32;
   return num_cus == kPipeXcds * 32 && g1.engine != GemmEngine::kTile && g2.engine != GemmEngine::kTile &&
          g1.route_in_kernel == 1 && g1.sw.enabled && g1.num_experts <= kFusedMaxExperts &&
-         (whole_chunks || pipe_small(g1)) &&
+         (whole_chunks || pipe_small(g1)) && reinterpret_cast<uintptr_t>(g1.sw.y) % 128 == 0 &&
          c1.ring[0] == kStreamDepth && c1.ring[1] == kStreamDepth && c2.ring[0] == kStreamDepth &&
          c2.ring[1] == kStreamDepth && stream_chunk(g1.k, kAChunk / 64, kNarrowDepth) > 0 &&
          g2.k <= kPipeMaxInter && c2.kc[0] == g2.k && 2 * c2.kc[1] >= g2.k && g2.k % (64 * kNarrowDepth) == 0 &&

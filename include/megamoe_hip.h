@@ -138,7 +138,8 @@ typedef struct mmoe_forward_args {
   const void* w2;                    /* e4m3 Marlin [E, H/16, I*16] */
   const float* w2_sf;                /* f32 [E, H] */
   int32_t* stats;                    /* int32 [E] or NULL (accumulated) */
-  void* route_scratch;               /* device workspace, >= mmoe_route_scratch_bytes() */
+  void* route_scratch;               /* device workspace, >= mmoe_route_scratch_bytes(); best on a
+                                        128-byte boundary (mmoe_forward) */
   int64_t route_scratch_bytes;
   int64_t sym_buffer_bytes;          /* size of the buffer x/x_sf/topk_* live in (checked) */
   const int32_t* runtime_num_tokens; /* device int32 [1] or NULL: tokens read at run time */
@@ -187,7 +188,9 @@ const char* mmoe_status_string(int status);
  * the 256-CU MI355X) the layer is one persistent launch whose workgroups hand rows to each other
  * through bounded waits: it needs the whole GPU, and a wait that runs out (another kernel
  * holding CUs for longer than the bound) leaves a wrong y. The launch still ends, and the call's
- * status (mmoe_scratch_status) is nonzero then. */
+ * status (mmoe_scratch_status) is nonzero then. The one launch needs route_scratch on a 128-byte
+ * boundary (any allocation is); a call whose route_scratch lies elsewhere runs a launch for each
+ * stage, with the same results. */
 int mmoe_forward(const mmoe_forward_args* args, void* stream);
 
 /* Status of the last mmoe_forward / mmoe_forward_static call on route_scratch (NULL: the static

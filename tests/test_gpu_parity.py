@@ -888,6 +888,33 @@ def test_caller_scratch_reused_across_shapes(mm, cuda, full_weights):
         assert torch.equal(y.view(torch.int16), y_ref.view(torch.int16)), f"S={s}: output"
 
 
+@pytest.mark.parametrize("offset", [128, 64, 16])
+@pytest.mark.parametrize("s", [40, 300])
+def test_caller_scratch_off_a_line_boundary(mm, cuda, full_weights, s, offset):
+    """A route_scratch off the 128-byte boundary: two groups' y rows would share a line there, which
+    the decode pipeline's hand-off does not allow, so the call runs the separate launches (nothing
+    writes the pipeline's row maxima); on the boundary it runs the pipeline. Bitwise the same y."""
+    import ctypes
+
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the decode pipeline runs on the whole 256-CU MI355X only")
+    l1, l2 = full_weights[0], full_weights[1]
+    log(f"scratch at a line's byte {offset % 128}, S={s}")
+    buf = mm.get_symm_buffer_for_mega_moe(None, 32, s, 6, 4096, 2048)
+    y_ref = run_layer(mm, buf, *make_tokens(s, 4096, 32, 6, seed=s), l1, l2).clone()
+    rows, n = int(buf.scratch_view("meta")[0].item()), buf.route_scratch.numel()
+    scratch = torch.zeros((n + 128,), dtype=torch.int8, device=cuda)[offset:offset + n]
+    assert scratch.data_ptr() % 128 == offset % 128
+    buf.route_scratch = scratch
+    buf.scratch_view("pmax").fill_(-1.0)
+    y = torch.full((s, 4096), 7.0, dtype=torch.bfloat16, device=cuda)
+    mm.fp8_w8a8_mega_moe(y, l1, l2, buf)
+    torch.cuda.synchronize()
+    assert bool((buf.scratch_view("pmax")[:rows] >= 0).all()) == (offset == 128), "which launches ran"
+    assert torch.all(buf.scratch_view("pipe").cpu() == 0) and mm.last_call_status(buf) == 0
+    assert torch.equal(y.view(torch.int16), y_ref.view(torch.int16))
+
+
 def test_layer_no_routed_rows(mm, cuda):
     """Every slot invalid -> y == 0 exactly (no partial contributes)."""
     s, e, hdim, inter = 10, 4, 256, 128
