@@ -85,14 +85,28 @@ __device__ __forceinline__ v16f mfma_fp8(const v8i& a, const v8i& b, const v16f&
   return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
 }
 
-// c += a b with the accumulator in AGPRs. Inline assembly: from the builtin the register allocator
-// moved some of a tile's 64 accumulators through VGPRs in the loop. The compiler does not see the
-// instruction's latency: read accumulators only after mfma_settle.
-__device__ __forceinline__ void mfma_fp8_16(const v8i& a, const v8i& b, v4f& c) {
-  asm("v_mfma_f32_16x16x128_f8f6f4 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+// c[n] += b[n] a for the four 16-column tiles n of an MFMA group, the accumulators in AGPRs. Inline
+// assembly: from the builtin the register allocator moved some of a tile's 64 accumulators through
+// VGPRs in the loop. The compiler adds no wait states to instructions that it does not see:
+//  * an operand that a VALU instruction has written (a copy that the compiler puts in front of the
+//    block) may be read two wait states later at the earliest. The block holds no s_nop for that: with
+//    one in front of each group (or MFMA) a layer of 24.7K rows takes 690 us instead of 683 and one of
+//    196K rows 4995 instead of 4946, and the operands come straight from memory and LDS;
+//  * no accumulator may be read or copied between a group and mfma_settle.
+// tests/test_isa_waits.py checks both in the code as built, along every path.
+__device__ __forceinline__ void mfma_group(const v8i (&b)[4], const v8i& a, v4f (&c)[4]) {
+  asm volatile(
+      "v_mfma_f32_16x16x128_f8f6f4 %0, %4, %8, %0\n\t"
+      "v_mfma_f32_16x16x128_f8f6f4 %1, %5, %8, %1\n\t"
+      "v_mfma_f32_16x16x128_f8f6f4 %2, %6, %8, %2\n\t"
+      "v_mfma_f32_16x16x128_f8f6f4 %3, %7, %8, %3"
+      : "+a"(c[0]), "+a"(c[1]), "+a"(c[2]), "+a"(c[3])
+      : "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "v"(a));
 }
 
-// The last MFMA's result (8 passes of 4 cycles) is in its registers before any of c is read.
+// The last MFMA's result (8 passes of 4 cycles) is in its registers before any of c is read. Volatile
+// like the groups, so the wait stays behind the last of them; every later read of c then depends on the
+// empty blocks, which stay behind the wait.
 template <int N>
 __device__ __forceinline__ void mfma_settle(v4f (&c)[N][4]) {
   asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
@@ -974,9 +988,9 @@ __device__ void wide_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, 
           load_b((ph + 2) % 3, j, min(kt + 2, last_stage));
       }
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn)
-        mfma_fp8_16(make_v8i(br[ph][tn][0], br[ph][tn][1]), abuf[gi % (kAhead + 1)], acc[gi][tn]);  // transposed tile
+      const v8i b[TN] = {make_v8i(br[ph][0][0], br[ph][0][1]), make_v8i(br[ph][1][0], br[ph][1][1]),
+                         make_v8i(br[ph][2][0], br[ph][2][1]), make_v8i(br[ph][3][0], br[ph][3][1])};
+      mfma_group(b, abuf[gi % (kAhead + 1)], acc[gi]);  // transposed tile
       __builtin_amdgcn_sched_barrier(0);
     }
     lds_barrier();
