@@ -65,6 +65,7 @@ constexpr int kStreamAutoMaxRows = kStreamItemRows;  // the auto schedule stream
 constexpr int kStreamDepth = 4;     // 64-k weight steps in flight per wave
 constexpr int kAChunk = 65536;      // bytes of one A chunk buffer (32*MT rows x 2048/MT k)
 constexpr int kALoads = kAChunk / 1024 / kGemmWaves;  // 16-byte A loads per lane per chunk
+constexpr int kTailDepth = 2;       // the same with a short last chunk (StreamTail)
 constexpr int kNarrowDepth = 8;     // weight steps in flight of a narrow item's waves
 constexpr int kAChunk4 = kAChunk / 256;  // k-bytes of a chunk of 128 rows in half a buffer
 // TILE engine: 256 x 256 output tile, BK = 128, the 8 waves as 2 (M) x 4 (N), each wave 128
@@ -364,19 +365,22 @@ struct AChunk {
 // kNarrow: only the first `waves` waves have columns (2 or 4 of the 8); the others help with A
 // and leave. A ring of 8 steps then keeps enough bytes in flight, and the few waves need no
 // barrier a step.
+// kTail: kc need not divide K (both are multiples of 64*D, and kc <= K). A last chunk that is shorter is
+// loaded as the last kc bytes of K: its steps are the end of what lies in LDS, and no load is masked.
 struct NoHook {
   __device__ __forceinline__ void operator()() const {}
 };
 template <bool kGather, bool kSwiglu, int MT, int D, bool kEarly = false, bool kAResident = false,
           bool kPmax = false, bool kCoherent = false, bool kNarrow = false, int kLoads = kALoads,
-          typename Hook = NoHook>
+          bool kTail = false, typename Hook = NoHook>
 __device__ void stream_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, int mrows, int nb,
                             int kc, uint8_t* smem, TileTables& tt, const Hook& before_a = Hook{},
                             int waves = kGemmWaves) {
   static_assert(!kAResident || kEarly, "a resident A is staged by the hook");
   using Chunk = AChunk<MT, kLoads>;
   const int spc = kc / 64;  // steps per chunk
-  const int nchunks = g.k / kc;
+  const int nchunks = kTail ? (g.k + kc - 1) / kc : g.k / kc;
+  const int last_spc = kTail ? g.k / 64 - (nchunks - 1) * spc : spc;  // steps of the last chunk
   const int tid = opaque_tid();
   const int lane = tid & (kWave - 1);
   const int wave = tid / kWave;
@@ -398,7 +402,7 @@ __device__ void stream_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0
   auto load_chunk = [&](int chunk) {
     if constexpr (kAResident) return;
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) astage[i] = ld16(asrc[i] + static_cast<int64_t>(chunk) * kc);
+    for (int i = 0; i < kLoads; ++i) astage[i] = ld16(asrc[i] + (kTail ? min(chunk * kc, g.k - kc) : static_cast<int64_t>(chunk) * kc));
   };
   auto store_chunk = [&](int chunk) {
     if constexpr (kAResident) return;
@@ -513,11 +517,11 @@ __device__ void stream_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0
     lds_barrier();
   }
   {
-    const int c = nchunks - 1;
-    for (int j = 0; j + D < spc; j += D) {
+    const int c = nchunks - 1, j0 = spc - last_spc;
+    for (int j = 0; j + D < last_spc; j += D) {
 #pragma unroll
       for (int d = 0; d < D; ++d) {
-        compute(d, c, j + d);
+        compute(d, c, j0 + j + d);
         issue(d, c * spc + j + d + D);
         __builtin_amdgcn_sched_barrier(0);
         if (!kNarrow) step_barrier();
@@ -1304,16 +1308,24 @@ __device__ __forceinline__ void tile_coords(int local, int cnt, int tile_nb, int
   mt = group * 4 + (in_group - nb * rows_in_group);
 }
 
-// kAnyK: K whose STREAM chunks do not take the 4-step weight ring (K not a multiple of 256); the
-// other shapes compile without those variants, which keeps the kernel's code (and its cold
-// instruction fetches in the one-time prologue) smaller.
+// kTail (stream_tail): how the STREAM engine cuts K. Kernels of their own, so that a kernel's code (and its
+// cold instruction fetches in the one-time prologue) holds one ring for each item height, and because
+// the short last chunk costs the ring of 4 ten spilled registers (K = 3072 and 1024, 256 tokens on 32
+// experts: 71 -> 76 us a layer).
+//   kNone: chunks that divide K, rings of 4
+//   k256: K a multiple of 256; chunks with a short last one and a ring of 2 up to 64 rows, chunks of 256
+//     and a ring of 4 above
+//   kAnyK: chunks with a short last one and a ring of 2
+enum class StreamTail { kNone, k256, kAnyK };
+
 // A dual launch's kernel that the routed rows do not select returns at once (GemmArgs).
 __device__ __forceinline__ bool dual_skips(const GemmArgs& g, bool wide) {
   return g.dual_rows != nullptr && ((*g.dual_rows >= g.dual_min_rows) != wide);
 }
 
-template <bool kGather, bool kSwiglu, bool kAnyK>
+template <bool kGather, bool kSwiglu, StreamTail kTail>
 __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs g) {
+  constexpr int kRing = kTail == StreamTail::kNone ? kStreamDepth : kTailDepth;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   __shared__ int s_prefix[kMaxGemmExperts + 1];
   __shared__ int s_tile[kMaxGemmExperts];
@@ -1414,15 +1426,14 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs 
         rs = RowSrc{s_tok, s_rw, row0};
       }
       if (mrows > 64) {
-        if (!kAnyK || g.ring[2] == 4)
-          stream_tile<kGather, kSwiglu, 4, 4, false, false, false, false, false, kALoads / 2>(g, rs, e, row0, mrows, nb, kAChunk4, smem, s_tt);
-        else if (kAnyK) stream_tile<kGather, kSwiglu, 4, 2>(g, rs, e, row0, mrows, nb, g.kc[2], smem, s_tt);
+        if constexpr (kTail != StreamTail::kAnyK)
+          stream_tile<kGather, kSwiglu, 4, kStreamDepth, false, false, false, false, false, kALoads / 2>(g, rs, e, row0, mrows, nb, kAChunk4, smem, s_tt);
+        else
+          stream_tile<kGather, kSwiglu, 4, kTailDepth, false, false, false, false, false, kALoads, true>(g, rs, e, row0, mrows, nb, g.kc[2], smem, s_tt);
       } else if (mrows > 32) {
-        if (!kAnyK || g.ring[1] == 4) stream_tile<kGather, kSwiglu, 2, 4>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
-        else if (kAnyK) stream_tile<kGather, kSwiglu, 2, 2>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
+        stream_tile<kGather, kSwiglu, 2, kRing, false, false, false, false, false, kALoads, kTail != StreamTail::kNone>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
       } else {
-        if (!kAnyK || g.ring[0] == 4) stream_tile<kGather, kSwiglu, 1, 4>(g, rs, e, row0, mrows, nb, g.kc[0], smem, s_tt);
-        else if (kAnyK) stream_tile<kGather, kSwiglu, 1, 2>(g, rs, e, row0, mrows, nb, g.kc[0], smem, s_tt);
+        stream_tile<kGather, kSwiglu, 1, kRing, false, false, false, false, false, kALoads, kTail != StreamTail::kNone>(g, rs, e, row0, mrows, nb, g.kc[0], smem, s_tt);
       }
     }
     __syncthreads();
@@ -2103,10 +2114,10 @@ hipError_t launch_wide(const GemmArgs& g, int max_rows, int num_cus, hipStream_t
                        dim3(kWideThreads), W::kSmemBytes, stream, g);
 }
 
-template <bool kGather, bool kSwiglu, bool kAnyK>
+template <bool kGather, bool kSwiglu, StreamTail kTail>
 hipError_t launch_engines_k(const GemmArgs& g, int max_rows, int num_cus, hipStream_t stream) {
   {  // the 128 KB of dynamic LDS exceeds the default limit
-    const hipError_t err = ensure_dynamic_lds<&grouped_gemm_kernel<kGather, kSwiglu, kAnyK>>(kSmemBytes);
+    const hipError_t err = ensure_dynamic_lds<&grouped_gemm_kernel<kGather, kSwiglu, kTail>>(kSmemBytes);
     if (err != hipSuccess) return err;
   }
   // upper bound of the work items over any split of max_rows rows into the experts
@@ -2119,41 +2130,59 @@ hipError_t launch_engines_k(const GemmArgs& g, int max_rows, int num_cus, hipStr
                                                         : std::max(stream_items, tile_items);
   int64_t grid = num_cus;  // one 8-wave workgroup per CU
   if (grid > bound) grid = bound;
-  return launch_kernel(grouped_gemm_kernel<kGather, kSwiglu, kAnyK>, dim3(static_cast<unsigned>(grid)),
+  return launch_kernel(grouped_gemm_kernel<kGather, kSwiglu, kTail>, dim3(static_cast<unsigned>(grid)),
                        dim3(kGemmThreads), kSmemBytes, stream, g);
 }
 
-// The largest multiple of 64 * steps that divides k and is at most cap; 0: there is none.
-int stream_chunk(int k, int cap, int steps) {
-  for (int kc = cap / (64 * steps) * (64 * steps); kc > 0; kc -= 64 * steps)
+// The largest multiple of 64 * ring that divides k and is at most cap; 0: there is none.
+int whole_chunk(int k, int cap, int ring) {
+  for (int kc = cap / (64 * ring) * (64 * ring); kc > 0; kc -= 64 * ring)
     if (k % kc == 0) return kc;
   return 0;
 }
 
-// The STREAM engine's chunks of K for 1, 2 and 4 row tiles: as long as the LDS buffers allow, so that
-// the workgroup's barriers are few, with a ring of 4 weight steps unless a ring of 2 makes a chunk at
-// least twice as long (K not a multiple of 256: 640 = 10 steps). Beside the accumulators of 4 row
+// The chunk of the fewest, about equally long, chunks of k that are at most cap each and whole rings (k
+// and cap are multiples of 64 * ring); the last one may be shorter.
+int tail_chunk(int k, int cap, int ring) {
+  const int unit = 64 * ring, chunks = (k + cap - 1) / cap;
+  return (k + chunks * unit - 1) / (chunks * unit) * unit;
+}
+
+// The LDS buffer of a chunk of MT = 1 << i row tiles, in k-bytes.
+int chunk_cap(int i) { return kAChunk / 32 >> i; }
+
+// The STREAM engine's chunks of K for 1, 2 and 4 row tiles with a ring of 4 weight steps: as long as
+// the LDS buffers allow, so that the workgroup's barriers are few. Beside the accumulators of 4 row
 // tiles a ring of 4 leaves registers for half the A loads only, so chunks of 256 in half the buffers:
 // 2715 rows of 32 experts 181.5 -> 177 us a layer against a ring of 2 and chunks of 512.
 void set_stream_chunks(GemmArgs* g) {
-  for (int i = 0; i < 2; ++i) {
-    const int cap = kAChunk / 32 >> i;
-    const int four = stream_chunk(g->k, cap, kStreamDepth);
-    const int two = stream_chunk(g->k, cap, 2);
-    g->ring[i] = 2 * four > two ? kStreamDepth : 2;
-    g->kc[i] = 2 * four > two ? four : two;
-  }
-  g->ring[2] = g->k % kAChunk4 == 0 ? kStreamDepth : 2;
-  g->kc[2] = g->k % kAChunk4 == 0 ? kAChunk4 : stream_chunk(g->k, kAChunk / 128, 2);
+  for (int i = 0; i < 2; ++i) g->kc[i] = whole_chunk(g->k, chunk_cap(i), kStreamDepth);
+  g->kc[2] = kAChunk4;
+}
+
+// A short last chunk where K is not a multiple of 256, or where chunks that divide K are at most half as
+// long: a chunk's loads and LDS writes are those of a whole buffer, and every chunk ends in a barrier.
+// 256 tokens on 32 experts, top-6 of 128 (I = 1024 where K = H, H = 4096 where K = I), us a layer, chunks
+// of 128 or 256 / the kernel here: K = H = 2944 90 / 71, 4352 115 / 104, 5504 203 / 192; K = I = 2176 188 /
+// 182.
+StreamTail stream_tail(const GemmArgs& g) {
+  if (g.k % (64 * kStreamDepth) != 0) return StreamTail::kAnyK;
+  for (int i = 0; i < 2; ++i)
+    if (2 * whole_chunk(g.k, chunk_cap(i), kStreamDepth) <= tail_chunk(g.k, chunk_cap(i), kTailDepth)) return StreamTail::k256;
+  return StreamTail::kNone;
 }
 
 template <bool kGather, bool kSwiglu>
 hipError_t launch_engines(const GemmArgs& args, int max_rows, int num_cus, hipStream_t stream) {
   GemmArgs g = args;
-  set_stream_chunks(&g);
-  return g.ring[0] == 4 && g.ring[1] == 4 && g.ring[2] == 4
-             ? launch_engines_k<kGather, kSwiglu, false>(g, max_rows, num_cus, stream)
-             : launch_engines_k<kGather, kSwiglu, true>(g, max_rows, num_cus, stream);
+  const StreamTail tail = stream_tail(g);
+  if (tail == StreamTail::kNone) {
+    set_stream_chunks(&g);
+    return launch_engines_k<kGather, kSwiglu, StreamTail::kNone>(g, max_rows, num_cus, stream);
+  }
+  for (int i = 0; i < 3; ++i) g.kc[i] = tail_chunk(g.k, chunk_cap(i), kTailDepth);
+  return tail == StreamTail::k256 ? launch_engines_k<kGather, kSwiglu, StreamTail::k256>(g, max_rows, num_cus, stream)
+                                  : launch_engines_k<kGather, kSwiglu, StreamTail::kAnyK>(g, max_rows, num_cus, stream);
 }
 
 }  // namespace
@@ -2226,12 +2255,14 @@ bool decode_pipeline_supported(const GemmArgs& g1, const GemmArgs& g2, int num_c
   GemmArgs c1 = g1, c2 = g2;
   set_stream_chunks(&c1);
   set_stream_chunks(&c2);
+  for (int i = 0; i < 2; ++i)  // (chunks that a ring of 2 steps would not make twice as long)
+    if (2 * c1.kc[i] <= whole_chunk(g1.k, chunk_cap(i), 2) || 2 * c2.kc[i] <= whole_chunk(g2.k, chunk_cap(i), 2))
+      return false;
   const bool whole_chunks = g1.k % (kAChunk / 32) == 0 && g2.k == kAChunk / 32;
   return num_cus == kPipeXcds * 32 && g1.engine != GemmEngine::kTile && g2.engine != GemmEngine::kTile &&
          g1.route_in_kernel == 1 && g1.sw.enabled && g1.num_experts <= kFusedMaxExperts &&
          (whole_chunks || pipe_small(g1)) && reinterpret_cast<uintptr_t>(g1.sw.y) % 128 == 0 &&
-         c1.ring[0] == kStreamDepth && c1.ring[1] == kStreamDepth && c2.ring[0] == kStreamDepth &&
-         c2.ring[1] == kStreamDepth && stream_chunk(g1.k, kAChunk / 64, kNarrowDepth) > 0 &&
+         whole_chunk(g1.k, kAChunk / 64, kNarrowDepth) > 0 &&
          g2.k <= kPipeMaxInter && c2.kc[0] == g2.k && 2 * c2.kc[1] >= g2.k && g2.k % (64 * kNarrowDepth) == 0 &&
          g1.n == 2 * g1.sw.inter && g2.k == g1.sw.inter && g1.n % (kStreamUnit * kGemmWaves) == 0 &&
          g2.n % (kStreamUnit * kGemmWaves) == 0 && g1.row_token != nullptr && g2.row_token == nullptr &&
@@ -2250,7 +2281,7 @@ hipError_t launch_decode_pipeline(const PipeArgs& args, int num_cus, hipStream_t
   PipeArgs p = args;
   set_stream_chunks(&p.g1);
   set_stream_chunks(&p.g2);
-  p.narrow_kc1 = stream_chunk(p.g1.k, kAChunk / 64, kNarrowDepth);
+  p.narrow_kc1 = whole_chunk(p.g1.k, kAChunk / 64, kNarrowDepth);
   return launch_kernel(small ? decode_pipeline_kernel<true> : decode_pipeline_kernel<false>,
                        dim3(static_cast<unsigned>(num_cus)), dim3(kGemmThreads), kSmemBytes, stream, p);
 }

@@ -91,10 +91,9 @@ struct GemmArgs {
   int num_experts;
   int n;
   int k;
-  // the STREAM engine's k-bytes a chunk and weight steps in flight for items of 1, 2 and 4 row tiles
-  // of 32 (set by the launch functions)
+  // the STREAM engine's k-bytes a chunk for items of 1, 2 and 4 row tiles of 32 (set by the launch
+  // functions)
   int kc[3];
-  int ring[3];
   GemmEngine engine;
   SwigluEpilogue sw;         // GEMM1 only (requires row_token); c is unused then
   int route_in_kernel;       // GEMM1: 1 = route the tasks in the kernel (<= gemm_route_max_tasks()),

@@ -851,6 +851,37 @@ def test_decode_pipeline_small_other_shapes(mm, cuda, hdim, inter, s):
     assert O.calc_diff(y.cpu(), tr.y) <= CALC_DIFF_BAR
 
 
+@pytest.mark.parametrize("hdim,inter", [(2944, 1408), (4352, 2176), (1408, 2816), (640, 4352)])
+def test_stream_chunks_with_a_short_last_one(mm, cuda, hdim, inter):
+    """STREAM items of 1, 2 and 4 row tiles at K whose chunks end in a short one (K = 128 and 256 times a
+    prime, in GEMM1 and in GEMM2): the stages against the oracle, and y bitwise that of the TILE engine,
+    which has no chunks."""
+    import ctypes
+
+    counts = (1, 32, 33, 64, 65, 128, 0, 20)
+    idx = torch.cat([torch.full((n,), i, dtype=torch.int64) for i, n in enumerate(counts)])
+    gen = torch.Generator().manual_seed(hdim)
+    idx = idx[torch.randperm(idx.numel(), generator=gen)].view(-1, 1).contiguous()
+    s, e = idx.shape[0], len(counts)
+    w = torch.rand((s, 1), generator=gen) + 0.05
+    x_fp8, x_sf = O.cast_to_fp8_channelwise(torch.randn((s, hdim), generator=gen).to(torch.bfloat16))
+    l1, l2 = make_weights_gpu(e, hdim, inter, seed=inter, mm=mm)
+    buf = mm.SymmBuffer(None, e, s, 1, hdim, inter)
+    log(f"STREAM chunks H={hdim} I={inter} S={s}")
+    buf.scratch_view("pmax").fill_(-1.0)
+    y = run_layer(mm, buf, x_fp8, x_sf, idx, w, l1, l2)
+    torch.cuda.synchronize()
+    assert buf.scratch_view("meta")[1].item() == 0 and bool((buf.scratch_view("pmax") < 0).all()), "the 8-wave kernel"
+    tr = O.mega_moe_forward(x_fp8, x_sf, idx, w, *cpu_weights(l1, l2))
+    _stage_checks(buf, tr, s)
+    _combine_bitwise(mm, buf, y, l1, l2, s, None)
+    assert O.calc_diff(y.cpu(), tr.y) <= CALC_DIFF_BAR
+    y_tile = torch.empty_like(y)
+    args = mm._forward_args(y_tile, l1, l2, None, buf, None, mm._capi.MMOE_SCHEDULE_STAGED)
+    assert mm._capi.load().mmoe_forward(ctypes.byref(args), mm._stream_handle()) == 0
+    assert torch.equal(y.view(torch.int16), y_tile.view(torch.int16))
+
+
 def test_caller_scratch_reused_across_shapes(mm, cuda, full_weights):
     """One caller-owned route_scratch, zero-filled once, serves mmoe_forward calls of different
     shapes in turn through the C ABI: an all-local 1024-token call (6144 rows: its y spans
