@@ -1585,19 +1585,31 @@ __device__ void pipe_combine_token(const PipeArgs& p, int64_t t, const uint8_t* 
 // of 2, 4 or 8 units, else chunks of up to 128 rows in GEMM1 and of 64 rows in GEMM2 (whose A rows
 // are resident in LDS) and whole items.
 //
-// 64-column units (waves) of an item of the small kernel when there are G groups: the widest items
-// that still give most CUs one. A CU reads at most ~50 GB/s, so ~140 of them saturate the HBM, and
-// whole items (8 waves) do that from 17 groups on; with fewer groups the same columns go to more CUs
-// in narrower items. At least 2: the 64 channels that two units of GEMM1 write to a row of y are one
-// 128-byte line, which then comes from one workgroup. 6 rows on 6 experts (4096 x 4096 and 4096 x
-// 2048): 66 us with 48 of the 256 CUs on whole items, 34 us with items of 2 units on 192.
+// 64-column units (waves) of an item of the small kernel in a GEMM of n columns when there are G groups:
+// the widest items of which there are still kFullItems. A CU reads at most ~50 GB/s, so ~140 of them
+// saturate the HBM, and whole items (8 waves) do that from 17 groups of 4096 columns on; with fewer items
+// the same columns go to more CUs in narrower ones. At least 2: the 64 channels that two units of GEMM1
+// write to a row of y are one 128-byte line, which then comes from one workgroup. 6 rows on 6 experts at
+// H = 4096, I = 2048: 66 us with 48 of the 256 CUs on whole items, 38 us with items of 2 units on 192.
+// Against whole items from 17 groups on in any GEMM: 318 rows on 32 experts at H = 4096, I = 512 70 -> 49
+// us, at H = 2048, I = 1024 56 -> 48; 10 rows at H = 7168, I = 2048 64 -> 58.
+constexpr int kFullItems = 136;
+
 template <bool kSmall>
 struct PipeShape {
   static constexpr int kRows1 = kSmall ? 32 : kStreamItemRows;  // rows of a GEMM1 item (a group)
   static constexpr int kRows2 = kSmall ? 32 : kStreamRows;      // rows of a GEMM2 item
   static_assert(kRows1 % kRows2 == 0, "a GEMM2 item's rows are one group's");
-  static __device__ __forceinline__ int units(int G) { return !kSmall || G > 16 ? kGemmWaves : G > 8 ? 4 : 2; }
+  static constexpr __host__ __device__ int units(int G, int n) {
+    const int all = G * (n / kStreamUnit);
+    return !kSmall || all >= 8 * kFullItems ? kGemmWaves : all >= 4 * kFullItems ? 4 : 2;
+  }
 };
+static_assert(PipeShape<true>::units(17, 4096) == 8 && PipeShape<true>::units(16, 4096) == 4 &&
+                  PipeShape<true>::units(8, 4096) == 2,
+              "4096 columns: whole items from 17 groups on");
+static_assert(PipeShape<true>::units(40, 1024) == 4 && PipeShape<true>::units(10, 7168) == 8,
+              "the width follows the items that the GEMM makes, not the groups");
 
 // Wave 0: s_prefix[0..E] = exclusive prefix of the experts' chunks of `rows` rows; their number.
 __device__ int plan_chunks(int E, int rows, const int* s_count, int* s_prefix) {
@@ -1815,8 +1827,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
   const bool too_many = s_prefix1[E] > kMaxPipeGroups;
   if (too_many && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&p.pipe[kPipeFailAt], 1);
   const int G = __builtin_amdgcn_readfirstlane(too_many ? 0 : s_prefix1[E]);
-  const int waves = Shape::units(G);
-  const int n1 = g1.n / (kStreamUnit * waves), n2 = g2.n / (kStreamUnit * waves);
+  const int waves1 = Shape::units(G, g1.n), waves2 = Shape::units(G, g2.n);
+  const int n1 = g1.n / (kStreamUnit * waves1), n2 = g2.n / (kStreamUnit * waves2);
   // Whole groups to an XCD, one group's items after the other's, when a last round of GEMM1 items keeps
   // at most half of the CUs: the others go on to GEMM2 meanwhile, and the groups of the rounds before
   // are complete then. Dealt item by item, a group's items can lie in two XCDs' ranges, and column block
@@ -1889,8 +1901,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
                      nb == 0 ? r0 + rows1 : 0, 0, 0, s_task, s_tok, s_rw);
         };
         const RowSrc rs{s_tok, s_rw, row0};
-        if (kSmall && waves < kGemmWaves)
-          stream_tile<true, true, 1, kNarrowDepth, true, false, true, true, true, kALoads / 2>(q.g1, rs, e, row0, mrows, nb, q.narrow_kc1, smem, s_tt, rank_rows, waves);
+        if (kSmall && waves1 < kGemmWaves)
+          stream_tile<true, true, 1, kNarrowDepth, true, false, true, true, true, kALoads / 2>(q.g1, rs, e, row0, mrows, nb, q.narrow_kc1, smem, s_tt, rank_rows, waves1);
         else if (!kSmall && mrows > 64)
           stream_tile<true, true, 4, 2, true, false, true, true, false, kALoads / 2>(q.g1, rs, e, row0, mrows, nb, kAChunk4, smem, s_tt, rank_rows);
         else if (!kSmall && mrows > 32)
@@ -1913,8 +1925,8 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
           __syncthreads();
         };
         const RowSrc rs{nullptr, nullptr, 0};
-        if (kSmall && waves < kGemmWaves)
-          stream_tile<false, false, 1, kNarrowDepth, true, true, false, true, true>(q.g2, rs, e, row0, mrows, nb, q.g2.kc[0], smem, s_tt, stage_rows, waves);
+        if (kSmall && waves2 < kGemmWaves)
+          stream_tile<false, false, 1, kNarrowDepth, true, true, false, true, true>(q.g2, rs, e, row0, mrows, nb, q.g2.kc[0], smem, s_tt, stage_rows, waves2);
         else if (!kSmall && mrows > 32)
           stream_tile<false, false, 2, kStreamDepth, true, true, false, true>(q.g2, rs, e, row0, mrows, nb, q.g2.kc[1], smem, s_tt, stage_rows);
         else

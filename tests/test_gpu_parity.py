@@ -830,10 +830,11 @@ def test_decode_pipeline_item_shapes(mm, cuda, full_weights, case):
         assert torch.all(buf.scratch_view("pipe").cpu() == 0), "counters"
 
 
-@pytest.mark.parametrize("hdim,inter,s", [(7168, 2048, 16), (4096, 1536, 24), (2560, 512, 40), (640, 768, 30)])
+@pytest.mark.parametrize("hdim,inter,s", [(7168, 2048, 16), (4096, 1536, 24), (2560, 512, 40), (640, 768, 30),
+                                           (7168, 512, 20), (1024, 512, 40), (512, 2048, 40)])
 def test_decode_pipeline_small_other_shapes(mm, cuda, hdim, inter, s):
     """The small kernel at other expert shapes (K in chunks that are not the LDS buffers' whole
-    length), and a hidden size it does not take (640: the separate launches)."""
+    length; items of another width in GEMM1 than in GEMM2), and a hidden size it does not take (640: the separate launches)."""
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the decode pipeline runs on the whole 256-CU MI355X only")
     e, k = 16, 8
