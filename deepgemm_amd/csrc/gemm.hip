@@ -1611,6 +1611,21 @@ static_assert(PipeShape<true>::units(17, 4096) == 8 && PipeShape<true>::units(16
 static_assert(PipeShape<true>::units(40, 1024) == 4 && PipeShape<true>::units(10, 7168) == 8,
               "the width follows the items that the GEMM makes, not the groups");
 
+// Whole groups to an XCD, one group's items after the other's, when a last round of GEMM1 items keeps at most
+// half of the CUs: the others go on to GEMM2 meanwhile, and the groups of the rounds before are complete
+// then. Dealt item by item, a group's items can lie in two XCDs' ranges, and column block by column block
+// an expert's groups end together: the first GEMM2 items then wait for the last round (1560, 1800 and 2040
+// Zipf rows: 198, 197 and 197 us; whole groups 184, 185 and 187). Above half, and when the last round is
+// full, the even deal ends the last round earlier (2160, 2400 and 2640 rows: 199, 201 and 200 us; whole
+// groups 204, 213 and 217; 64 groups, two full rounds, 3666 and 3634 rows: 214 and 238 against 231 and 246).
+constexpr __host__ __device__ bool few_in_last_round(int items, int cus) {
+  const int last = items % cus;
+  return items > cus && last != 0 && 2 * last <= cus;
+}
+static_assert(few_in_last_round(384, 256) && !few_in_last_round(392, 256) && !few_in_last_round(512, 256) &&
+                  !few_in_last_round(256, 256) && few_in_last_round(264, 256),
+              "a full last round is not a short one");
+
 // Wave 0: s_prefix[0..E] = exclusive prefix of the experts' chunks of `rows` rows; their number.
 __device__ int plan_chunks(int E, int rows, const int* s_count, int* s_prefix) {
   const int lane = lane_id();
@@ -1829,16 +1844,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
   const int G = __builtin_amdgcn_readfirstlane(too_many ? 0 : s_prefix1[E]);
   const int waves1 = Shape::units(G, g1.n), waves2 = Shape::units(G, g2.n);
   const int n1 = g1.n / (kStreamUnit * waves1), n2 = g2.n / (kStreamUnit * waves2);
-  // Whole groups to an XCD, one group's items after the other's, when a last round of GEMM1 items keeps
-  // at most half of the CUs: the others go on to GEMM2 meanwhile, and the groups of the rounds before
-  // are complete then. Dealt item by item, a group's items can lie in two XCDs' ranges, and column block
-  // by column block an expert's groups end together: the first GEMM2 items then wait for the last round
-  // (1560, 1800 and 2040 Zipf rows: 198, 197 and 197 us; whole groups 184, 185 and 187). Above half, the even
-  // deal ends the last round earlier (2160, 2400 and 2640 rows: 199, 201 and 200 us; whole groups 204, 213
-  // and 217).
-  const int items1 = G * n1, last_round = items1 % static_cast<int>(gridDim.x);
-  const bool by_group = items1 > static_cast<int>(gridDim.x) && 2 * last_round <= static_cast<int>(gridDim.x) &&
-                        s_rows1 == Shape::kRows2;
+  const bool by_group = few_in_last_round(G * n1, static_cast<int>(gridDim.x)) && s_rows1 == Shape::kRows2;
   const float* task_w = reinterpret_cast<const float*>(smem);  // valid until the first item's loads
   bool first_item = true;
   for (int phase = 0; phase < 2; ++phase) {
