@@ -308,7 +308,8 @@ __global__ __launch_bounds__(kEltThreads) void gather_tasks_kernel(uint8_t* gx, 
 
 // The rows that the routing may leave out (counts above the tasks' own): weight 0, expert -1.
 __global__ __launch_bounds__(kEltThreads) void clear_rows_kernel(float* row_weight, int32_t* m_indices, int rows) {
-  for (int r = blockIdx.x * kEltThreads + threadIdx.x; r < rows; r += gridDim.x * kEltThreads) {
+  // (64-bit: the step past the last row of a count near 2^31 does not fit an int)
+  for (int64_t r = blockIdx.x * kEltThreads + threadIdx.x; r < rows; r += gridDim.x * kEltThreads) {
     row_weight[r] = 0.0f;
     m_indices[r] = -1;
   }

@@ -1437,6 +1437,26 @@ def test_deepep_preprocess_no_tokens(mm, cuda):
         assert torch.all(rw == 0) and torch.all(mi == -1)
 
 
+def test_deepep_preprocess_clears_every_row_of_the_largest_count(mm, cuda):
+    """The most rows that the count's type holds, without a received token: every row reads weight 0
+    and expert -1 (the row after the last step of a thread is past 2^31)."""
+    import ctypes
+
+    rows, lib = 2 ** 31 - 1, mm._capi.load()
+    log(f"preprocess clears {rows} rows")
+    w = torch.full((rows,), 7.0, dtype=torch.float32, device=cuda)
+    m = torch.full((rows,), 7, dtype=torch.int32, device=cuda)
+    need = ctypes.c_int64()
+    assert lib.mmoe_deepep_preprocess_workspace_bytes(0, 4, 8, rows, ctypes.byref(need)) == 0
+    assert lib.mmoe_deepep_preprocess_channelwise(
+        None, None, w.data_ptr(), m.data_ptr(), None, None, None, None, None, None, rows, 0, 4, 256, 8, 1,
+        None, need.value, mm._stream_handle()) == 0
+    for part in range(0, rows, 1 << 28):
+        assert bool((w[part:part + (1 << 28)] == 0).all()) and bool((m[part:part + (1 << 28)] == -1).all())
+    del w, m
+    torch.cuda.empty_cache()
+
+
 def test_api_flag_and_tensor_errors(mm, cuda, monkeypatch):
     """The reference's flag and tensor checks raise the same exception types and messages
     (megamoe/__init__.py:343-410, csrc/apis/mega_dcu.hpp:355-433, large_opt.py:381, :526,
