@@ -585,7 +585,7 @@ int mmoe_deepep_preprocess_workspace_bytes(int recv_rows, int topk, int num_expe
   off = align_up(off + (num_experts + 1) * 4, 256);      // offsets
   off = align_up(off + 16 * 4, 256);                     // meta
   off = align_up(off + mmoe::route_count_ints(tasks, num_experts) * 4, 256);  // chunk, wave counts
-  off = align_up(off + (total_rows > 0 ? total_rows : 1) * 4, 256);  // row_token
+  off = align_up(off + (total_rows > 0 ? total_rows : 1) * int64_t{4}, 256);  // row_token
   *out_bytes = off;
   return MMOE_OK;
 }
@@ -631,7 +631,7 @@ int mmoe_deepep_preprocess_channelwise(void* grouped_x, float* grouped_x_scale,
   r.meta = at<int32_t>(workspace, take(16 * 4));
   r.chunk_counts = at<int32_t>(workspace, take(mmoe::route_count_ints(tasks, num_experts) * 4));
   r.wave_counts = r.chunk_counts + (chunks > 0 ? chunks : 1) * num_experts;
-  r.row_token = at<int32_t>(workspace, take((total_rows > 0 ? total_rows : 1) * 4));
+  r.row_token = at<int32_t>(workspace, take((total_rows > 0 ? total_rows : 1) * int64_t{4}));
   r.topk_idx = recv_topk_ids;
   r.idx_i64 = topk_ids_i64 ? 1 : 0;
   r.topk_w = recv_topk_weights;

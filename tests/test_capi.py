@@ -183,6 +183,14 @@ def test_forward_zero_tokens_is_a_noop():
     assert lib.mmoe_forward(ctypes.byref(_args(num_tokens=0)), None) == 0
 
 
+@pytest.mark.parametrize("rows", [1, 2 ** 29, 2 ** 31 - 1])
+def test_preprocess_workspace_holds_every_row(rows):
+    """The preprocess workspace holds a token index for each row, also where its bytes pass 2^31."""
+    need = ctypes.c_int64()
+    assert _capi.load().mmoe_deepep_preprocess_workspace_bytes(16, 4, 8, rows, ctypes.byref(need)) == 0
+    assert 4 * rows <= need.value <= 4 * rows + (1 << 16)
+
+
 def test_check_raises_runtime_error():
     with pytest.raises(RuntimeError, match="too many tokens"):
         _capi.check(-6, "fp8_mega_moe")
