@@ -65,8 +65,7 @@ def test_cast_fp8_channelwise_every_kernel(mm, cuda, cols):
     zeros the same from both kernels."""
     bits = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
     finite = bits[torch.isfinite(bits)]
-    finite = finite[finite.abs() < 2.0 ** 120]
-    rows = min(200, -(-finite.numel() // cols))
+    rows = -(-finite.numel() // cols)
     gen = torch.Generator().manual_seed(cols)
     # ascending in magnitude, so that a row's values span few binades and fill the codes
     finite = finite[finite.abs().float().argsort()]
