@@ -1586,15 +1586,13 @@ __device__ void pipe_combine_token(const PipeArgs& p, int64_t t, const uint8_t* 
 // are resident in LDS) and whole items.
 //
 // 64-column units (waves) of an item of the small kernel in a GEMM of n columns when there are G groups:
-// the widest items of which there are still kFullItems. A CU reads at most ~50 GB/s, so ~140 of them
-// saturate the HBM, and whole items (8 waves) do that from 17 groups of 4096 columns on; with fewer items
-// the same columns go to more CUs in narrower ones. At least 2: the 64 channels that two units of GEMM1
-// write to a row of y are one 128-byte line, which then comes from one workgroup. 6 rows on 6 experts at
-// H = 4096, I = 2048: 66 us with 48 of the 256 CUs on whole items, 38 us with items of 2 units on 192.
-// Against whole items from 17 groups on in any GEMM: 318 rows on 32 experts at H = 4096, I = 512 70 -> 49
-// us, at H = 2048, I = 1024 56 -> 48; 10 rows at H = 7168, I = 2048 64 -> 58.
-constexpr int kFullItems = 136;
-
+// the narrowest of 2, 4 and 8 whose items still are one round on the CUs. A CU reads at most ~50 GB/s, so
+// few items leave the HBM idle; a second round of narrow items costs more than it gains. At least 2: the
+// 64 channels that two units of GEMM1 write to a row of y are one 128-byte line, which then comes from one
+// workgroup. Us a layer of 8 rows a group with 2, 4 and 8 units in both GEMMs: H = 4096, I = 2048 47, 53,
+// 75 at 8 groups; 73, 56, 76 at 9; 83, 74, 85 at 16; 101, 103, 88 at 17. By each GEMM's own items: H =
+// 4096, I = 1536 47 at 9 groups (52, 54, 76), 77 at 21 (88, 81, 89), 89 at 22 (96, 95, 90); H = 7168,
+// I = 2048 58 at 5 (64, 73, 110).
 template <bool kSmall>
 struct PipeShape {
   static constexpr int kRows1 = kSmall ? 32 : kStreamItemRows;  // rows of a GEMM1 item (a group)
@@ -1602,14 +1600,15 @@ struct PipeShape {
   static_assert(kRows1 % kRows2 == 0, "a GEMM2 item's rows are one group's");
   static constexpr __host__ __device__ int units(int G, int n) {
     const int all = G * (n / kStreamUnit);
-    return !kSmall || all >= 8 * kFullItems ? kGemmWaves : all >= 4 * kFullItems ? 4 : 2;
+    return !kSmall || all > 4 * kPipeCus ? kGemmWaves : all > 2 * kPipeCus ? 4 : 2;
   }
 };
 static_assert(PipeShape<true>::units(17, 4096) == 8 && PipeShape<true>::units(16, 4096) == 4 &&
-                  PipeShape<true>::units(8, 4096) == 2,
+                  PipeShape<true>::units(9, 4096) == 4 && PipeShape<true>::units(8, 4096) == 2,
               "4096 columns: whole items from 17 groups on");
-static_assert(PipeShape<true>::units(40, 1024) == 4 && PipeShape<true>::units(10, 7168) == 8,
-              "the width follows the items that the GEMM makes, not the groups");
+static_assert(PipeShape<true>::units(32, 1024) == 2 && PipeShape<true>::units(10, 7168) == 8 &&
+                  PipeShape<true>::units(21, 3072) == 4 && PipeShape<true>::units(22, 3072) == 8,
+              "the width follows the items that the GEMM makes, not the groups, and keeps them one round");
 
 // Whole groups to an XCD, one group's items after the other's, when a last round of GEMM1 items keeps at most
 // half of the CUs: the others go on to GEMM2 meanwhile, and the groups of the rounds before are complete
@@ -1618,12 +1617,12 @@ static_assert(PipeShape<true>::units(40, 1024) == 4 && PipeShape<true>::units(10
 // Zipf rows: 198, 197 and 197 us; whole groups 184, 185 and 187). Above half, and when the last round is
 // full, the even deal ends the last round earlier (2160, 2400 and 2640 rows: 199, 201 and 200 us; whole
 // groups 204, 213 and 217; 64 groups, two full rounds, 3666 and 3634 rows: 214 and 238 against 231 and 246).
-constexpr __host__ __device__ bool few_in_last_round(int items, int cus) {
-  const int last = items % cus;
-  return items > cus && last != 0 && 2 * last <= cus;
+constexpr __host__ __device__ bool few_in_last_round(int items) {
+  const int last = items % kPipeCus;
+  return items > kPipeCus && last != 0 && 2 * last <= kPipeCus;
 }
-static_assert(few_in_last_round(384, 256) && !few_in_last_round(392, 256) && !few_in_last_round(512, 256) &&
-                  !few_in_last_round(256, 256) && few_in_last_round(264, 256),
+static_assert(few_in_last_round(384) && !few_in_last_round(392) && !few_in_last_round(512) && !few_in_last_round(256) &&
+                  few_in_last_round(264),
               "a full last round is not a short one");
 
 // Wave 0: s_prefix[0..E] = exclusive prefix of the experts' chunks of `rows` rows; their number.
@@ -1844,7 +1843,7 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
   const int G = __builtin_amdgcn_readfirstlane(too_many ? 0 : s_prefix1[E]);
   const int waves1 = Shape::units(G, g1.n), waves2 = Shape::units(G, g2.n);
   const int n1 = g1.n / (kStreamUnit * waves1), n2 = g2.n / (kStreamUnit * waves2);
-  const bool by_group = few_in_last_round(G * n1, static_cast<int>(gridDim.x)) && s_rows1 == Shape::kRows2;
+  const bool by_group = few_in_last_round(G * n1) && s_rows1 == Shape::kRows2;
   const float* task_w = reinterpret_cast<const float*>(smem);  // valid until the first item's loads
   bool first_item = true;
   for (int phase = 0; phase < 2; ++phase) {
@@ -2277,7 +2276,7 @@ bool decode_pipeline_supported(const GemmArgs& g1, const GemmArgs& g2, int num_c
     if (2 * c1.kc[i] <= whole_chunk(g1.k, chunk_cap(i), 2) || 2 * c2.kc[i] <= whole_chunk(g2.k, chunk_cap(i), 2))
       return false;
   const bool whole_chunks = g1.k % (kAChunk / 32) == 0 && g2.k == kAChunk / 32;
-  return num_cus == kPipeXcds * 32 && g1.engine != GemmEngine::kTile && g2.engine != GemmEngine::kTile &&
+  return num_cus == kPipeCus && g1.engine != GemmEngine::kTile && g2.engine != GemmEngine::kTile &&
          g1.route_in_kernel == 1 && g1.sw.enabled && g1.num_experts <= kFusedMaxExperts &&
          (whole_chunks || pipe_small(g1)) && reinterpret_cast<uintptr_t>(g1.sw.y) % 128 == 0 &&
          whole_chunk(g1.k, kAChunk / 64, kNarrowDepth) > 0 &&

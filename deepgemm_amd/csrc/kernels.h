@@ -207,6 +207,7 @@ hipError_t launch_combine(const CombineArgs& c, int num_cus, hipStream_t stream)
 // kMaxPipeGroups) and GEMM2 items done per expert (expert e's at kPipeDone2At + e *
 // kPipeDone2Stride: the combine's waves poll them).
 constexpr int kPipeXcds = 8;
+constexpr int kPipeCus = kPipeXcds * 32;  // workgroups: the pipeline runs on the whole MI355X only
 constexpr int kPipeLine = 32;
 constexpr int kPipeClaim2 = kPipeLine / 2;
 constexpr int kPipeExitAt = (kPipeXcds + 1) * kPipeLine;
