@@ -268,7 +268,7 @@ const char* mmoe_build_config(void) {
          "\"weight_scale_mode\": \"channelwise_fp32\", \"input_scale_mode\": "
          "\"channelwise_fp32\", \"l2_act_scale_mode\": \"channelwise_fp32\", "
          "\"has_fp8_api\": true, \"has_fp4_api\": false, \"mfma\": "
-         "\"v_mfma_f32_32x32x64_f8f6f4\", \"fusion_boundary\": "
+         "\"v_mfma_f32_32x32x64_f8f6f4, v_mfma_f32_16x16x128_f8f6f4\", \"fusion_boundary\": "
          "\"route|gemm1(gather)|swiglu_quant|gemm2|combine\", \"num_ranks\": 1}";
 }
 
@@ -336,8 +336,8 @@ int mmoe_forward_stages(const mmoe_forward_args* a, int first_stage, int last_st
   const int max_rows = a->num_tokens * a->num_topk;
   void* ws = a->route_scratch;
 
-  // Small task counts: GEMM1 routes in-kernel (one launch fewer, no single-workgroup routing
-  // latency); the routing kernels serve larger counts and a routing-only call.
+  // Small task counts: GEMM1 routes in-kernel (one launch fewer); the routing kernels serve larger
+  // counts and a routing-only call.
   const bool route_in_gemm1 = runs(MMOE_STAGE_ROUTE) && runs(MMOE_STAGE_GEMM1) &&
                               max_rows <= mmoe::gemm_route_max_tasks() &&
                               a->num_experts <= mmoe::gemm_route_max_experts();

@@ -36,11 +36,12 @@
 //    - TILE engine (more rows). A 256 x 256 output tile per workgroup, the 8 waves as 2 x 4
 //      with 128 x 64 each, K in 128-byte stages through double-buffered LDS (A rows
 //      XOR-swizzled, B in Marlin's own 256-byte blocks).
-//    Both engines use the 32x32x64 MFMA, let lane l supply k-bytes [32*(l/32), 32*(l/32)+32) of each 64-k MFMA step
-//    for A and B alike and accumulate the 64-k steps in the same order.
+//    Both engines use the 32x32x64 MFMA, let lane l supply k-bytes [32*(l/32), 32*(l/32)+32) of each
+//    64-k MFMA step for A and B alike and accumulate the 64-k steps in the same order: the same bits.
 //  * the 4-wave WIDE kernel (every expert with many rows: prefill, MFMA-bound): one wave per
 //    SIMD with its 256 accumulators in AGPRs, 256 x 256 tiles of 16x16x128 MFMAs, weights straight
-//    into registers and only A through LDS; described at wide_tile.
+//    into registers and only A through LDS; described at wide_tile. Its sums take 128 products a step
+//    (nearly always the same bits).
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -65,7 +66,7 @@ constexpr int kStreamAutoMaxRows = kStreamItemRows;  // the auto schedule stream
 constexpr int kStreamDepth = 4;     // 64-k weight steps in flight per wave
 constexpr int kAChunk = 65536;      // bytes of one A chunk buffer (32*MT rows x 2048/MT k)
 constexpr int kALoads = kAChunk / 1024 / kGemmWaves;  // 16-byte A loads per lane per chunk
-constexpr int kTailDepth = 2;       // the same with a short last chunk (StreamTail)
+constexpr int kTailDepth = 2;       // the same with a short last chunk (stream_tail)
 constexpr int kNarrowDepth = 8;     // weight steps in flight of a narrow item's waves
 constexpr int kAChunk4 = kAChunk / 256;  // k-bytes of a chunk of 128 rows in half a buffer
 // TILE engine: 256 x 256 output tile, BK = 128, the 8 waves as 2 (M) x 4 (N), each wave 128
@@ -235,10 +236,8 @@ __device__ __forceinline__ void publish_tile_scales(TileTables& tt, const TileSc
 // the output (mrows <= 32 * MT; table row trow0 + r holds row r's scales), 64-column unit `unit`
 // of the output (SwiGLU: 32 channels).
 // kCoherent: the stores go out device-coherent (sc1, written through the XCD's L2): GEMM2's
-// partial rows, so that workgroups of other XCDs can read them in the same launch, and GEMM1's
-// SwiGLU rows of the decode pipeline, which its GEMM2 items of the same XCD still read from L2
-// but which no longer sit there dirty (c1 150.9 -> 148.9 us per layer; its y output rows written
-// through as well made no difference, its act rows as 4-byte coherent stores +3 us).
+// partial rows and GEMM1's SwiGLU rows in the decode pipeline, which workgroups of other XCDs read in
+// the same launch.
 // SwiGLU: y is stored in bf16 (the reference fused path's rounding of the activation before
 // its quantization). kPmax (the decode pipeline's GEMM1): the row maxima of the rounded values
 // are stored as well.
@@ -693,9 +692,10 @@ __device__ void tile_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, 
 //
 // The MFMA is 16x16x128. At these sizes the chip is power-bound, and it takes less power for a FLOP
 // than 32x32x64: register-only loops over random e4m3 values sustain 4.43 against 4.05 PFLOP/s (over
-// zeros 4.97 and 4.96). Here the clock rises from 1.9 to 2.0 GHz, and a layer of 24.7K rows (4096 x
-// 4096, 4096 x 2048) goes from 703 to 689 us, of 49K Zipf rows from 1268 to 1256, of 196K rows from
-// 4845 to 4822; the results are the same bits. A first version with a two-stage ring (one burst of
+// zeros 4.97 and 4.96). A layer of 24.7K rows (4096 x 4096, 4096 x 2048) goes from 703 to 689 us, of 49K
+// Zipf rows from 1268 to 1256, of 196K rows from 4845 to 4822. It adds 128 products a step where the
+// 8-wave engines' MFMA adds 64, so a sum can round differently in its last fp32 bit: about one bf16
+// partial value in 10^8 is another than theirs. A first version with a two-stage ring (one burst of
 // loads a stage) was 1-3% slower than 32x32x64. Where the cycles are, by timing copies at 196K
 // rows: GEMM1 5.65 M, without A's and B's loads 4.5 M, without the LDS reads too 4.4 M (prologues and
 // epilogues then are 1.25 M of it), 3.15 M of MFMA.
@@ -1312,20 +1312,20 @@ __device__ __forceinline__ void tile_coords(int local, int cnt, int tile_nb, int
 // cold instruction fetches in the one-time prologue) holds one ring for each item height, and because
 // the short last chunk costs the ring of 4 ten spilled registers (K = 3072 and 1024, 256 tokens on 32
 // experts: 71 -> 76 us a layer).
-//   kNone: chunks that divide K, rings of 4
-//   k256: K a multiple of 256; chunks with a short last one and a ring of 2 up to 64 rows, chunks of 256
+//   kTailNone: chunks that divide K, rings of 4
+//   kTail256: K a multiple of 256; chunks with a short last one and a ring of 2 up to 64 rows, chunks of 256
 //     and a ring of 4 above
-//   kAnyK: chunks with a short last one and a ring of 2
-enum class StreamTail { kNone, k256, kAnyK };
+//   kTailAny: chunks with a short last one and a ring of 2
+constexpr int kTailNone = 0, kTail256 = 1, kTailAny = 2;
 
 // A dual launch's kernel that the routed rows do not select returns at once (GemmArgs).
 __device__ __forceinline__ bool dual_skips(const GemmArgs& g, bool wide) {
   return g.dual_rows != nullptr && ((*g.dual_rows >= g.dual_min_rows) != wide);
 }
 
-template <bool kGather, bool kSwiglu, StreamTail kTail>
+template <bool kGather, bool kSwiglu, int kTail>
 __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs g) {
-  constexpr int kRing = kTail == StreamTail::kNone ? kStreamDepth : kTailDepth;
+  constexpr int kRing = kTail == kTailNone ? kStreamDepth : kTailDepth;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   __shared__ int s_prefix[kMaxGemmExperts + 1];
   __shared__ int s_tile[kMaxGemmExperts];
@@ -1426,14 +1426,14 @@ __global__ __launch_bounds__(kGemmThreads, 1) void grouped_gemm_kernel(GemmArgs 
         rs = RowSrc{s_tok, s_rw, row0};
       }
       if (mrows > 64) {
-        if constexpr (kTail != StreamTail::kAnyK)
+        if constexpr (kTail != kTailAny)
           stream_tile<kGather, kSwiglu, 4, kStreamDepth, false, false, false, false, false, kALoads / 2>(g, rs, e, row0, mrows, nb, kAChunk4, smem, s_tt);
         else
           stream_tile<kGather, kSwiglu, 4, kTailDepth, false, false, false, false, false, kALoads, true>(g, rs, e, row0, mrows, nb, g.kc[2], smem, s_tt);
       } else if (mrows > 32) {
-        stream_tile<kGather, kSwiglu, 2, kRing, false, false, false, false, false, kALoads, kTail != StreamTail::kNone>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
+        stream_tile<kGather, kSwiglu, 2, kRing, false, false, false, false, false, kALoads, kTail != kTailNone>(g, rs, e, row0, mrows, nb, g.kc[1], smem, s_tt);
       } else {
-        stream_tile<kGather, kSwiglu, 1, kRing, false, false, false, false, false, kALoads, kTail != StreamTail::kNone>(g, rs, e, row0, mrows, nb, g.kc[0], smem, s_tt);
+        stream_tile<kGather, kSwiglu, 1, kRing, false, false, false, false, false, kALoads, kTail != kTailNone>(g, rs, e, row0, mrows, nb, g.kc[0], smem, s_tt);
       }
     }
     __syncthreads();
@@ -1812,8 +1812,9 @@ __global__ __launch_bounds__(kGemmThreads, 1) void decode_pipeline_kernel(PipeAr
   if (threadIdx.x < kWave) {
     fused_scan(E, s_wcnt, s_count, s_off);
     // groups of GEMM2's rows when they take no more rounds of items than the larger ones: an item of 4
-    // row tiles has half the weight steps in flight (2046 Zipf rows: 217 us in 128-row groups, 199
-    // in 64-row ones, both two rounds; 3072 even rows, one round against two: 203 and 223)
+    // row tiles has half the weight steps in flight (three loads of 2046 Zipf rows: 207-216 us in
+    // 128-row groups, 186-194 in 64-row ones, both two rounds; 3072 even rows, one round against two: 203
+    // and 223)
     const int n = stream_blocks(g1), cus = static_cast<int>(gridDim.x);
     int rows = Shape::kRows1;
     const int chunks1 = plan_chunks(E, rows, s_count, s_prefix1);
@@ -2131,7 +2132,7 @@ hipError_t launch_wide(const GemmArgs& g, int max_rows, int num_cus, hipStream_t
                        dim3(kWideThreads), W::kSmemBytes, stream, g);
 }
 
-template <bool kGather, bool kSwiglu, StreamTail kTail>
+template <bool kGather, bool kSwiglu, int kTail>
 hipError_t launch_engines_k(const GemmArgs& g, int max_rows, int num_cus, hipStream_t stream) {
   {  // the 128 KB of dynamic LDS exceeds the default limit
     const hipError_t err = ensure_dynamic_lds<&grouped_gemm_kernel<kGather, kSwiglu, kTail>>(kSmemBytes);
@@ -2182,24 +2183,24 @@ void set_stream_chunks(GemmArgs* g) {
 // 256 tokens on 32 experts, top-6 of 128 (I = 1024 where K = H, H = 4096 where K = I), us a layer, chunks
 // of 128 or 256 / the kernel here: K = H = 2944 90 / 71, 4352 115 / 104, 5504 203 / 192; K = I = 2176 188 /
 // 182.
-StreamTail stream_tail(const GemmArgs& g) {
-  if (g.k % (64 * kStreamDepth) != 0) return StreamTail::kAnyK;
+int stream_tail(const GemmArgs& g) {
+  if (g.k % (64 * kStreamDepth) != 0) return kTailAny;
   for (int i = 0; i < 2; ++i)
-    if (2 * whole_chunk(g.k, chunk_cap(i), kStreamDepth) <= tail_chunk(g.k, chunk_cap(i), kTailDepth)) return StreamTail::k256;
-  return StreamTail::kNone;
+    if (2 * whole_chunk(g.k, chunk_cap(i), kStreamDepth) <= tail_chunk(g.k, chunk_cap(i), kTailDepth)) return kTail256;
+  return kTailNone;
 }
 
 template <bool kGather, bool kSwiglu>
 hipError_t launch_engines(const GemmArgs& args, int max_rows, int num_cus, hipStream_t stream) {
   GemmArgs g = args;
-  const StreamTail tail = stream_tail(g);
-  if (tail == StreamTail::kNone) {
+  const int tail = stream_tail(g);
+  if (tail == kTailNone) {
     set_stream_chunks(&g);
-    return launch_engines_k<kGather, kSwiglu, StreamTail::kNone>(g, max_rows, num_cus, stream);
+    return launch_engines_k<kGather, kSwiglu, kTailNone>(g, max_rows, num_cus, stream);
   }
   for (int i = 0; i < 3; ++i) g.kc[i] = tail_chunk(g.k, chunk_cap(i), kTailDepth);
-  return tail == StreamTail::k256 ? launch_engines_k<kGather, kSwiglu, StreamTail::k256>(g, max_rows, num_cus, stream)
-                                  : launch_engines_k<kGather, kSwiglu, StreamTail::kAnyK>(g, max_rows, num_cus, stream);
+  return tail == kTail256 ? launch_engines_k<kGather, kSwiglu, kTail256>(g, max_rows, num_cus, stream)
+                          : launch_engines_k<kGather, kSwiglu, kTailAny>(g, max_rows, num_cus, stream);
 }
 
 }  // namespace
@@ -2249,11 +2250,19 @@ bool gemm_eager_dual(const GemmArgs& g, int max_rows) {
          static_cast<int64_t>(max_rows) < 8ll * kStreamAutoMaxRows * g.num_experts;
 }
 
-// Tasks (S * K) up to which the pipeline's small kernel runs. At 4096 x 4096 and 4096 x 2048, top-6,
-// 32 of 256 experts local: 34 against 70 us on the large one at 8 tokens, 56 / 77 at 24, 90 / 96 at
-// 48; from ~22 experts with rows on they tie (64 tokens: 105 both). A chunk is 32 rows here, so a
-// skewed load past this bound pays for it: 80 tokens on 26 of 28 Zipf experts 178 against 135 us.
+// Tasks (S * K) up to which the pipeline's small kernel runs. H = 4096, I = 2048, top-6, us on it and on
+// the large one, three loads each: 32 of 256 experts local 33-46 against 65-74 at 8 tokens, 43-91 against
+// 73-91 at 24, 61-110 against 78-110 at 48; past the bound they tie (64 tokens: 88-118 both). A chunk is 32
+// rows here, so a skewed load pays for it: Zipf loads of 28 local experts 66-76 against 82-86 at 8 tokens
+// and 107-119 against 112-121 at 24, but at 53 114, 128 and 135 against 118, 122 and 131, and past the
+// bound, at 80, 162-177 against 130-138. At H = 7168, top-8, the other side is the separate launches: 51-97
+// against 107-126 at 10 tokens, 113-190 against 137-189 at 40; Zipf loads 148-172 against 144-168 at 10
+// and 192, 210 and 224 against 202, 203 and 215 at 40.
 constexpr int kPipeSmallTasks = 320;
+// The groups' counters: a group of the small kernel has a row at least, one of the large kernel is a whole
+// chunk of GEMM2's rows or an expert's last.
+static_assert(kPipeSmallTasks <= kMaxPipeGroups && kFusedMaxTasks / kStreamRows + kFusedMaxExperts <= kMaxPipeGroups,
+              "a counter for every group");
 
 static bool pipe_small(const GemmArgs& g1) {
   return static_cast<int64_t>(g1.route.host_tokens) * g1.route.topk <= kPipeSmallTasks;

@@ -217,7 +217,9 @@ constexpr int kPipeFailAt = kPipeExitAt + 1;
 // (meta[3], mmoe_scratch_status) then reports that its output is not valid.
 constexpr int kPipeSpinLimit = 1 << 20;
 constexpr int kPipeHeader = (kPipeXcds + 2) * kPipeLine;
-constexpr int kMaxPipeGroups = 512;  // groups of <= 64 rows: S*K <= 8192 rows over <= 255 experts
+// Groups (GEMM1 chunks of an expert's rows): of <= 32 rows in the small kernel (S*K <= kPipeSmallTasks rows),
+// of <= 64 or 128 in the large one (S*K <= 8192 rows over <= 255 experts); gemm.hip asserts both bounds.
+constexpr int kMaxPipeGroups = 512;
 constexpr int kMaxPipeExperts = 256;
 constexpr int kPipeDone1At = kPipeHeader;
 constexpr int kPipeDone2At = kPipeHeader + kMaxPipeGroups;

@@ -659,6 +659,39 @@ def test_wide_tile_heights(mm, cuda, hdim, inter):
     assert O.calc_diff(y.cpu(), tr.y) <= CALC_DIFF_BAR
 
 
+def test_wide_and_streaming_sums_agree(mm, cuda, full_weights):
+    """The WIDE MFMA adds 128 products a step, the 8-wave engines' 64, so a sum can differ in its last
+    fp32 bit. One such bit in every sum would change one bf16 value in 2^16 by a bf16 step (1.5e-5 of
+    them); measured are about 1e-8. Compared over the SwiGLU rows and, where those are equal, GEMM2's
+    partial rows (all six slots of a token local, so every row has one)."""
+    import ctypes
+
+    l1, l2 = full_weights[0], full_weights[1]
+    s = 4096
+    log("WIDE against STREAM sums")
+    buf = mm.get_symm_buffer_for_mega_moe(None, 32, s, 6, 4096, 2048)
+    _load_bucket(buf, *make_tokens(s, 4096, 32, 6, seed=77))
+    rows = {}
+    for schedule in (mm._capi.MMOE_SCHEDULE_AUTO, mm._capi.MMOE_SCHEDULE_PERSISTENT):
+        y = torch.empty((s, 4096), dtype=torch.bfloat16, device=cuda)
+        args = mm._forward_args(y, l1, l2, None, buf, None, schedule)
+        assert mm._capi.load().mmoe_forward(ctypes.byref(args), mm._stream_handle()) == 0
+        torch.cuda.synchronize()
+        assert buf.scratch_view("meta")[1].item() == (schedule == mm._capi.MMOE_SCHEDULE_AUTO), "which GEMM1 ran"
+        r = buf.scratch_view("meta")[0].item()
+        rows[schedule] = [buf.scratch_view(n)[:r].clone() for n in ("y", "part")]
+    (y_w, part_w), (y_s, part_s) = rows.values()
+    y_diff = (y_w.view(torch.int16) != y_s.view(torch.int16))
+    assert y_diff.float().mean().item() <= 2.0 ** -16
+    same = ~y_diff.any(dim=1)
+    # (a zero's sign may differ: the WIDE epilogue writes -0 as +0)
+    a, b = part_w[same], part_s[same]
+    differ = a != b
+    assert differ.float().mean().item() <= 2.0 ** -16
+    step = (a.view(torch.int16).int() - b.view(torch.int16).int()).abs()[differ]
+    assert step.numel() == 0 or step.max().item() == 1, "by more than one bf16 step"
+
+
 def test_wide_token_matrix_over_4gb(mm, cuda):
     """A token matrix of more than 4 GB: the WIDE GEMM1 gathers its rows with 64-bit offsets.
     Sampled tokens at both ends and on both sides of the 4 GB line against the oracle."""
