@@ -82,9 +82,9 @@ def algorithmic_bytes(rows: int, touched: int) -> dict:
 
 # kernel names as rocprofv3 reports them: the 8-wave persistent kernel (decode-sized configs)
 # or the 4-wave WIDE kernel (many rows per expert)
-PROFILE_KERNELS = {"gemm1": ("grouped_gemm_kernel<true, true, false>", "wide_gemm_kernel<true, true, 256>"),
-                   "gemm2": ("grouped_gemm_kernel<false, false, false>", "wide_gemm_kernel<false, false, 256>"),
-                   "pipeline": ("decode_pipeline_kernel",)}
+PROFILE_KERNELS = {"gemm1": ("grouped_gemm_kernel<true, true, 0>", "wide_gemm_kernel<true, true, 256, false>"),
+                   "gemm2": ("grouped_gemm_kernel<false, false, 0>", "wide_gemm_kernel<false, false, 256, false>"),
+                   "pipeline": ("decode_pipeline_kernel<false>", "decode_pipeline_kernel<true>")}
 
 
 def profiled_traffic(config_id: str, kernel: str):

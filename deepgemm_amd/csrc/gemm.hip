@@ -693,7 +693,8 @@ __device__ void tile_tile(const GemmArgs& g, const RowSrc& rs, int e, int row0, 
 // The MFMA is 16x16x128. At these sizes the chip is power-bound, and it takes less power for a FLOP
 // than 32x32x64: register-only loops over random e4m3 values sustain 4.43 against 4.05 PFLOP/s (over
 // zeros 4.97 and 4.96). A layer of 24.7K rows (4096 x 4096, 4096 x 2048) goes from 703 to 689 us, of 49K
-// Zipf rows from 1268 to 1256, of 196K rows from 4845 to 4822. It adds 128 products a step where the
+// Zipf rows from 1268 to 1256, of 196K rows from 4845 to 4822: more cycles at a higher clock (counters
+// at 196K rows: GEMM1 5.5 M at 1.94 GHz, with 32x32x64 4.9 M at 1.75). It adds 128 products a step where the
 // 8-wave engines' MFMA adds 64, so a sum can round differently in its last fp32 bit: about one bf16
 // partial value in 10^8 is another than theirs. A first version with a two-stage ring (one burst of
 // loads a stage) was 1-3% slower than 32x32x64. Where the cycles are, by timing copies at 196K

@@ -47,3 +47,12 @@ def test_more_than_one_gpu_is_refused():
     assert res.returncode != 0
     assert "one GPU" in res.stdout + res.stderr
     assert res.stdout.strip() == "" or not res.stdout.lstrip().startswith("{")
+
+
+def test_profiled_traffic_is_found_for_every_profiled_config():
+    """The kernel names in the committed profiles are the ones that the bench looks for."""
+    for config, kernels in (("c1", ("pipeline",)), ("c2", ("gemm1", "gemm2")), ("c3", ("gemm1", "gemm2")),
+                            ("c4", ("gemm1", "gemm2")), ("m1", ("gemm1", "gemm2")), ("m2", ("gemm1", "gemm2"))):
+        for kernel in kernels:
+            traffic, path = bench.profiled_traffic(config, kernel)
+            assert traffic > 1 << 28 and config in path
